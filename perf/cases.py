@@ -114,8 +114,8 @@ def draw(rng):
         return {"kind": kind, "streams": _between(rng, 1, 16), "low": rng.randint(8, high),
                 "high": high, "prefix": rng.choice((0, 0, rng.randint(1, 700)))}
     if kind == "head":
-        return {"kind": kind, "streams": _between(rng, 1, 256)}
-    frames = _between(rng, 1, 400)
+        return {"kind": kind, "streams": _between(rng, 2, 256)}
+    frames = _between(rng, 3, 400)
     return {"kind": kind, "frames": frames, "chunk": max(-(-frames // 16), _between(rng, 1, frames))}
 
 
