@@ -389,6 +389,42 @@ def test_pcm_random_weights_against_oracle(lib, pkg, oracle, oracle_mod):
     p.close()
 
 
+@pytest.mark.parametrize("counts", [(1,) * 9, (2, 3, 4), (7, 2), (12, 20, 32), (33, 31)])
+def test_pcm_tile_shapes_and_passes(lib, pkg, oracle, oracle_mod, counts):
+    """Calls whose passes take each tile shape of the convolutions (from one
+    frame's 16 positions to a full pass, with remainders), and requests after a
+    reset: the bits of one frame at a time, whose first frames are the oracle's.
+    The state first runs another request, whose rows a new one must not see."""
+    mimi_w, convs = random_mimi(911), random_pcm_convs(912)
+    frames = sum(counts)
+    x = np.random.default_rng(913).standard_normal((frames, 32)).astype(np.float32)
+    views = pkg.Views()
+    p = Pcm(lib, pkg, views, mimi_w, convs)
+
+    def request(sizes):
+        lib.phonon_pcm_state_reset(p.h)
+        parts, off = [], 0
+        for n in sizes:
+            ok, raw, _ = p.process(x[off:off + n])
+            assert ok == 1
+            parts.append(raw)
+            off += n
+        return np.concatenate(parts)
+
+    assert p.process(x[::-1][:5])[0] == 1
+    single = request([1] * frames)
+    assert np.array_equal(request(counts), single)
+    known = min(frames, 4)
+    om = oracle_mod.MimiOracle(oracle, mimi_w)
+    oc = [oracle_mod.ConvOracle(oracle, w, b, s, t) for (w, b, s, t) in convs]
+    ok, exp = oracle_mod.pcm_process(oracle, om, oc, x[:known])
+    for c in oc:
+        c.close()
+    om.close()
+    assert ok and normwise(single[:known * 1920], exp) <= TOL
+    p.close()
+
+
 def test_pcm_rejects_bad_requests(lib, pkg):
     views = pkg.Views()
     p = Pcm(lib, pkg, views, mimi_identity_model(route_only=True), pcm_scalar_convs())
