@@ -1,6 +1,7 @@
-// Audio decoder kernels: the Mimi latent transformer's own steps
-// (src/phonon_mimi.c) and the SEANet convolutions (src/phonon_conv.c). The
-// Mimi projections run on the MFMA projection kernels (pgpu_gemm.hip).
+// Audio decoder kernels behind entry points of their own: the Mimi input and
+// RoPE steps (src/phonon_mimi.c) and single SEANet convolutions over fp32 rows
+// (src/phonon_conv.c). The latent-to-PCM decoder's products, attention and
+// residual pairs are in pgpu_pcm.hip.
 //
 // Every kernel works on all positions of a request at once: a causal
 // convolution's output position t reads the input window it needs, taking
@@ -50,17 +51,8 @@ __global__ __launch_bounds__(256) void k_mimi_input(const float *__restrict__ la
         hidden[((size_t)f * kMimiRows + o) * kWidth + c] = v;
     }
     flag_nonfinite(status, bad);
-    // Every block reads `previous` (f = 0 only) before any block writes it:
-    // the write is done by a separate launch (k_mimi_keep_previous).
-}
-
-__global__ void k_mimi_keep_previous(const float *__restrict__ latents, int frame,
-                                     const float *__restrict__ proj, float *__restrict__ previous) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    float dot = 0.0f;
-#pragma unroll 8
-    for (int i = 0; i < 32; i++) dot = dot + proj[c * 32 + i] * latents[frame * 32 + i];
-    previous[c] = dot;
+    // Only frame 0's work-groups read `previous`; the same threads replace it.
+    if (f == 0) previous[c] = frames > 1 ? project(frames - 1) : cur;
 }
 
 // RoPE of q and k of every row (position first + r), then k and v into the
@@ -91,123 +83,6 @@ __global__ __launch_bounds__(256) void k_mimi_rope_store(float *__restrict__ qkv
     }
     ring_v[slot + 2 * i] = row[2 * kWidth + 2 * i];
     ring_v[slot + 2 * i + 1] = row[2 * kWidth + 2 * i + 1];
-}
-
-// Windowed causal attention of one latent frame's 16 rows and one head per
-// work-group: row i (position p = first + 16 f + i) attends the keys of
-// positions max(0, p - context + 1) .. p. The frame's key window (at most
-// context + 15 positions) goes through LDS in chunks of 64 keys: scores
-// (one thread per (key, 4 rows), q . k over the 64 dimensions in order,
-// times 1/8), a masked softmax per row (one wave per 4 rows), then the
-// value sums (one thread per (dimension, 4 rows), keys in order), scaled
-// by 1/total at the end.
-constexpr int kAttnChunk = 64;
-constexpr int kAttnKeys = 256 + 16;  // context <= 256, plus the frame's rows
-
-__global__ __launch_bounds__(256) void k_mimi_attention(const float *__restrict__ qkv,
-                                                        long long first,
-                                                        const float *__restrict__ ring_k,
-                                                        const float *__restrict__ ring_v,
-                                                        int ring, int context,
-                                                        float *__restrict__ out, int *status) {
-    __shared__ float q[16][kHeadDim];
-    __shared__ float kv[kAttnChunk][kHeadDim + 1];
-    __shared__ float sc[16][kAttnKeys];
-    __shared__ float totals[16];
-    const int f = blockIdx.x, head = blockIdx.y, t = threadIdx.x;
-    const int wave = t >> 6, lane = t & 63;
-    const long long p0 = first + 16LL * f;
-    const long long kstart = p0 - (context - 1) > 0 ? p0 - (context - 1) : 0;
-    const int nkeys = (int)(p0 + 16 - kstart);
-    {
-        const int row = t >> 4, d = (t & 15) * 4;
-        const float4 v = *(const float4 *)(qkv + (size_t)(16 * f + row) * 3 * kWidth +
-                                           head * kHeadDim + d);
-        q[row][d] = v.x; q[row][d + 1] = v.y; q[row][d + 2] = v.z; q[row][d + 3] = v.w;
-    }
-    const int kk = t & 63, rg = (t >> 6) * 4;  // score / output thread roles
-    for (int c0 = 0; c0 < nkeys; c0 += kAttnChunk) {
-        {
-            const int key = t >> 2, d = (t & 3) * 16;
-            if (c0 + key < nkeys) {
-                const float4 *src = (const float4 *)(ring_k + (size_t)((kstart + c0 + key) % ring) *
-                                                                  kWidth + head * kHeadDim + d);
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const float4 v = src[u];
-                    kv[key][d + 4 * u] = v.x; kv[key][d + 4 * u + 1] = v.y;
-                    kv[key][d + 4 * u + 2] = v.z; kv[key][d + 4 * u + 3] = v.w;
-                }
-            }
-        }
-        __syncthreads();
-        if (c0 + kk < nkeys) {
-            const long long kpos = kstart + c0 + kk;
-            float dot[4] = {0.f, 0.f, 0.f, 0.f};
-            for (int d = 0; d < kHeadDim; d++) {
-                const float kd = kv[kk][d];
-#pragma unroll
-                for (int i = 0; i < 4; i++) dot[i] = dot[i] + q[rg + i][d] * kd;
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const long long p = p0 + rg + i;
-                sc[rg + i][c0 + kk] = kpos <= p && kpos > p - context ? dot[i] * 0.125f : -INFINITY;
-            }
-        }
-        __syncthreads();
-    }
-    // Masked softmax: wave w takes rows 4w .. 4w+3.
-    for (int i = 0; i < 4; i++) {
-        const int row = wave * 4 + i;
-        float mx = -INFINITY;
-        for (int j = lane; j < nkeys; j += 64) mx = fmaxf(mx, sc[row][j]);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-        float total = 0.0f;
-        for (int j = lane; j < nkeys; j += 64) {
-            const float s = sc[row][j];
-            const float e = s == -INFINITY ? 0.0f : expf(s - mx);
-            sc[row][j] = e;
-            total += e;
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
-        if (lane == 0) totals[row] = total;
-    }
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < nkeys; c0 += kAttnChunk) {
-        __syncthreads();  // scores final / previous chunk consumed
-        {
-            const int key = t >> 2, d = (t & 3) * 16;
-            if (c0 + key < nkeys) {
-                const float4 *src = (const float4 *)(ring_v + (size_t)((kstart + c0 + key) % ring) *
-                                                                  kWidth + head * kHeadDim + d);
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const float4 v = src[u];
-                    kv[key][d + 4 * u] = v.x; kv[key][d + 4 * u + 1] = v.y;
-                    kv[key][d + 4 * u + 2] = v.z; kv[key][d + 4 * u + 3] = v.w;
-                }
-            }
-        }
-        __syncthreads();
-        const int n = nkeys - c0 < kAttnChunk ? nkeys - c0 : kAttnChunk;
-        for (int j = 0; j < n; j++) {
-            const float vd = kv[j][kk];
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] = acc[i] + sc[rg + i][c0 + j] * vd;
-        }
-    }
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float total = totals[rg + i];
-        const float v = acc[i] * (1.0f / total);
-        out[(size_t)(16 * f + rg + i) * kWidth + head * kHeadDim + kk] = v;
-        bad |= !isfinite(v) || !(total > 0.0f);
-    }
-    flag_nonfinite(status, bad);
 }
 
 __device__ inline float elu1(float v) { return v <= 0.0f ? expf(v) - 1.0f : v; }
@@ -466,8 +341,6 @@ extern "C" int pgpu_mimi_input(void *stream, const float *latents, int frames,
     hipLaunchKernelGGL(k_mimi_input, dim3(frames, kWidth / 256), dim3(256), 0,
                        (hipStream_t)stream, latents, frames, projection, upsample, previous,
                        hidden, status);
-    hipLaunchKernelGGL(k_mimi_keep_previous, dim3(kWidth / 256), dim3(256), 0,
-                       (hipStream_t)stream, latents, frames - 1, projection, previous);
     return launch_ok("pgpu_mimi_input");
 }
 
@@ -480,17 +353,6 @@ extern "C" int pgpu_mimi_rope_store(void *stream, float *qkv, int rows, long lon
     hipLaunchKernelGGL(k_mimi_rope_store, dim3(rows), dim3(256), 0, (hipStream_t)stream, qkv,
                        rows, first, (const float2 *)rope, ring_k, ring_v, ring);
     return launch_ok("pgpu_mimi_rope_store");
-}
-
-extern "C" int pgpu_mimi_attention(void *stream, const float *qkv, int rows, long long first,
-                                   const float *ring_k, const float *ring_v, int ring,
-                                   int context, float *out, int *status) {
-    if (!qkv || rows <= 0 || rows % 16 || rows > 65535 || first < 0 || !ring_k || !ring_v ||
-        context <= 0 || context > 256 || ring < rows + context - 1 || !out || !status)
-        return bad_arguments("pgpu_mimi_attention");
-    hipLaunchKernelGGL(k_mimi_attention, dim3(rows / 16, kHeads), dim3(256), 0,
-                       (hipStream_t)stream, qkv, first, ring_k, ring_v, ring, context, out, status);
-    return launch_ok("pgpu_mimi_attention");
 }
 
 extern "C" int pgpu_conv_rows(void *stream, const pgpu_conv_layer *L, const float *x,

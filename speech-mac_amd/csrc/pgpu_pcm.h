@@ -32,22 +32,42 @@ typedef struct {
     int past;  /* 0: the request's first pass (what came before is zero) */
 } pgpu_pass;
 
-/* rows [positions][512] -> planes; positions >= 8. */
-int pgpu_pcm_rows_to_planes(void *stream, const float *rows, int positions, const pgpu_planes *out,
-                            pgpu_pass pass);
+/* LayerNorm of rows [positions][512] -> planes. */
+int pgpu_pcm_layer_norm(void *stream, const float *rows, const float *weight, const float *bias,
+                        float epsilon, int positions, const pgpu_planes *out, int *status);
 
-/* A convolution over planes: taps 7 (conv0: ncols = cout, ELU of the result
- * into `planes`) or taps 2 (a transposed convolution: ncols = stride * cout
- * columns k * cout + o per position, fp32 into `rows` [positions][ncols]).
- * in->channels is a multiple of 128, ncols and cout of 64; fragments as in
- * pgpu_conv_layer. positions >= 8. */
+/* A product over planes, and what becomes of it. in->channels is a multiple
+ * of 128 (512 for a projection), ncols of 64; fragments as in pgpu_conv_layer (a projection's
+ * pgpu_matrix values are the same records); positions >= 8.
+ *   ROWS   a transposed convolution: taps 2, ncols = stride * cout columns
+ *          k * cout + o, + bias, fp32 into rows [positions][ncols]
+ *   ELU    conv0: taps 7, + bias, ELU, into planes
+ *   GELU   a projection (taps 1), GELU, into planes
+ *   GATED  a projection to 512 columns: rows += gate * product, and, if
+ *          planes.data is set, the sum into planes too
+ *   QKV    the in-projection (1536 columns): RoPE of q and k at positions
+ *          first + r, q into rows [positions][512], k and v into their ring
+ *          slots (first + r) % ring */
+enum { PGPU_PLANE_ROWS, PGPU_PLANE_ELU, PGPU_PLANE_GELU, PGPU_PLANE_GATED, PGPU_PLANE_QKV };
 typedef struct {
-    int taps, ncols, cout;
+    int epilogue, ncols, cout;
     const uint16_t *fragments;
-    const float *bias;
-} pgpu_plane_conv;
-int pgpu_pcm_conv(void *stream, const pgpu_plane_conv *conv, const pgpu_planes *in, int positions,
-                  pgpu_pass pass, float *rows, const pgpu_planes *planes, int *status);
+    const float *bias; /* ROWS, ELU: [cout] */
+    const float *gate; /* GATED: [512] */
+    float *rows;
+    pgpu_planes planes;
+    const float *rope; /* QKV: [rope_positions][32] (cos, sin) */
+    long long first, rope_positions;
+    float *ring_k, *ring_v;
+    int ring;
+} pgpu_plane_product;
+int pgpu_pcm_product(void *stream, const pgpu_plane_product *product, const pgpu_planes *in,
+                     int positions, pgpu_pass pass, int *status);
+
+/* pgpu_mimi_attention with q as QKV leaves it and its rows into planes. */
+int pgpu_pcm_attention(void *stream, const float *q, int rows, long long first,
+                       const float *ring_k, const float *ring_v, int ring, int context,
+                       const pgpu_planes *out, int *status);
 
 /* A residual pair over x [positions][channels], channels 256, 128 or 64:
  * v = x + conv1(ELU(conv3(ELU(x)))). channels 256 and 128: ELU(v) into

@@ -1,6 +1,9 @@
-// The SEANet half of the latent-to-PCM decoder (src/phonon_pcm.c:145-170),
-// seven launches a pass: conv0, then per stage a transposed convolution and
-// its residual pair, the output convolution inside the last pair.
+// The latent-to-PCM decoder (src/phonon_mimi.c, src/phonon_pcm.c:145-170).
+// Mimi's two layers are six launches each (LayerNorm, in-projection with RoPE
+// and the ring, attention, out-projection, LayerNorm, the two MLP
+// projections), the SEANet half seven: conv0, then per stage a transposed
+// convolution and its residual pair, the output convolution inside the last
+// pair.
 //
 // What bounds it. Every product is fp32-accurate: a bf16 weight times the
 // three exact bf16 terms of an fp32 value, three matrix products. Splitting
@@ -9,14 +12,16 @@
 // that needs all of a position's channels anyway (the residual pairs, whose
 // hidden rows never leave LDS). A kernel that split its input for every tap
 // and column tile was bound by those instructions: its eleven launches took
-// 240 us per 32 frames and 155 us for one, these take 92 and 46 us.
+// 240 us per 32 frames and 155 us for one, these take 92 and 46 us. Mimi's
+// layers, with 16-position projection tiles and an attention on the vector
+// units before, went from 165 to 118 us per 32 frames and from 74 to 66 for one.
 //
-// Order of summation. k_conv_planes sums a fixed four ranges of input
+// Order of summation. k_plane_product sums a fixed four ranges of input
 // channels (one wave each; within one, 32-channel block by block, its taps in
 // order) and adds the four in order; the residual kernel runs one chain. No
 // output depends on the tile shape or on how many positions a pass has, so a
 // request gives the same bits however it is cut into calls.
-#include "pgpu_common.hpp"
+#include "pgpu_gemm.hpp"
 #include "pgpu_pcm.h"
 
 namespace pgpu {
@@ -54,16 +59,163 @@ __device__ inline void store_planes4(const pgpu_planes &out, int t, int position
     }
 }
 
-__global__ __launch_bounds__(256) void k_rows_to_planes(const float *__restrict__ rows,
-                                                        int positions, pgpu_planes out,
-                                                        int phase) {
-    // 16 positions x 16 groups of four channels per work-group.
-    const int t = blockIdx.x * 16 + (threadIdx.x & 15);
-    const int c = (blockIdx.y * 16 + (threadIdx.x >> 4)) * 4;
-    if (t >= positions) return;
-    const float4 v = *(const float4 *)(rows + (size_t)t * kWidth + c);
-    const float a[4] = {v.x, v.y, v.z, v.w};
-    store_planes4(out, t, positions, phase, c, a);
+// A wave normalises two rows with the decode step's LayerNorm arithmetic;
+// lane j holds channels 8j .. 8j + 7, a slot of each term. Four waves write
+// eight consecutive slots.
+__global__ __launch_bounds__(256) void k_ln_planes(const float *__restrict__ rows,
+                                                   const float *__restrict__ lw,
+                                                   const float *__restrict__ lb, float eps,
+                                                   int positions, pgpu_planes out, int *status) {
+    const int j = threadIdx.x & 63, t0 = blockIdx.x * 8 + (threadIdx.x >> 6) * 2;
+    Rows2 r;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        r.live[i] = t0 + i < positions;
+        const float *src = rows + (size_t)(r.live[i] ? t0 + i : positions - 1) * kWidth + j * 8;
+        const float4 a = *(const float4 *)src, b = *(const float4 *)(src + 4);
+        r.v[i][0] = a.x; r.v[i][1] = a.y; r.v[i][2] = a.z; r.v[i][3] = a.w;
+        r.v[i][4] = b.x; r.v[i][5] = b.y; r.v[i][6] = b.z; r.v[i][7] = b.w;
+    }
+    const bool bad = rows_ln_values(r, lw, lb, eps);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        if (!r.live[i]) continue;
+        uint16_t h[8], m[8], l[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) split3(r.v[i][e], h[e], m[e], l[e]);
+        uint4 *dst = (uint4 *)out.data + (size_t)j * out.stride + kSlots + t0 + i;
+        const size_t term = (size_t)(kWidth / 8) * out.stride;
+        dst[0] = uint4{pack16(h[0], h[1]), pack16(h[2], h[3]), pack16(h[4], h[5]),
+                       pack16(h[6], h[7])};
+        dst[term] = uint4{pack16(m[0], m[1]), pack16(m[2], m[3]), pack16(m[4], m[5]),
+                          pack16(m[6], m[7])};
+        dst[2 * term] = uint4{pack16(l[0], l[1]), pack16(l[2], l[3]), pack16(l[4], l[5]),
+                              pack16(l[6], l[7])};
+    }
+    flag_nonfinite(status, bad);
+}
+
+// Windowed causal attention of one latent frame's 16 rows and one head per
+// work-group (the contract of pgpu_mimi_attention). Both products run on the
+// fp32 matrix cores, whose operand layouts need no shuffles between them:
+// lane (g, n) = (lane / 16, lane % 16) of S^T = K Q^T holds keys 4g + r of
+// query n, which is the operand of O^T = V^T P^T when its step r takes keys
+// 4g + r. The window's up to 17 tiles of 16 keys go round the four waves;
+// every K and V value is loaded straight into its operand register, all of
+// them before the first product (one memory latency instead of one per
+// 64-key chunk, each behind a barrier; the products on the vector units took
+// most of 30 us per layer at 32 frames and 12 at one). Sums over the waves
+// go through LDS in wave order, so a row's bits depend on its position only.
+constexpr int kWaveTiles = 5;
+static_assert(4 * kWaveTiles * 16 >= 256 + 15, "four waves hold a frame's key window");
+
+template <bool PLANES>
+__global__ __launch_bounds__(256) void k_window_attention(
+    const float *__restrict__ q, int ld_q, long long first, const float *__restrict__ ring_k,
+    const float *__restrict__ ring_v, int ring, int context, float *__restrict__ rows,
+    pgpu_planes out, int positions, int *status) {
+    __shared__ float red[2][4][16];
+    __shared__ float4 part[4][4][64];
+    const int f = blockIdx.x, head = blockIdx.y;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const long long p0 = first + 16LL * f;
+    const long long kstart = p0 - (context - 1) > 0 ? p0 - (context - 1) : 0;
+    const int nkeys = (int)(p0 + 16 - kstart);  // <= 256 + 15
+    const int slot0 = (int)(kstart % ring);
+    auto slot = [&](int key) {
+        key = slot0 + (key < nkeys ? key : nkeys - 1);
+        return (size_t)(key < ring ? key : key - ring) * kWidth + head * kHeadDim;
+    };
+    float4 qv[4], kv[kWaveTiles][4], vv[kWaveTiles][4];
+    const float *qrow = q + (size_t)(16 * f + n) * ld_q + head * kHeadDim + 16 * g;
+#pragma unroll
+    for (int d = 0; d < 4; d++) qv[d] = *(const float4 *)(qrow + 4 * d);
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; i++) {
+        const float *src = ring_k + slot((wave + 4 * i) * 16 + n) + 16 * g;
+#pragma unroll
+        for (int d = 0; d < 4; d++) kv[i][d] = *(const float4 *)(src + 4 * d);
+    }
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            vv[i][r] = *(const float4 *)(ring_v + slot((wave + 4 * i) * 16 + 4 * g + r) + 4 * n);
+    f32x4 s[kWaveTiles];
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; i++) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < kWaveTiles; i++)
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float *)&kv[i][d])[e],
+                                                            ((const float *)&qv[d])[e], s[i], 0, 0,
+                                                            0);
+    // Masks and the softmax of query n.
+    const long long p = p0 + n;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const long long kp = kstart + (wave + 4 * i) * 16 + 4 * g + r;
+            s[i][r] = kp <= p && kp > p - context ? s[i][r] * 0.125f : -INFINITY;
+            mx = fmaxf(mx, s[i][r]);
+        }
+    mx = xor16_32_max(mx);
+    if (lane < 16) red[0][wave][lane] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0][0][n], red[0][1][n]), fmaxf(red[0][2][n], red[0][3][n]));
+    float total = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            s[i][r] = s[i][r] == -INFINITY ? 0.0f : expf(s[i][r] - mx);
+            total += s[i][r];
+        }
+    total = xor16_32_sum(total);
+    if (lane < 16) red[1][wave][lane] = total;
+    f32x4 o[4];
+#pragma unroll
+    for (int d = 0; d < 4; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kWaveTiles; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float *)&vv[i][r])[d],
+                                                            s[i][r], o[d], 0, 0, 0);
+    // o[d][r]: dimension 16 g + 4 r + d of query n. Wave w finishes r = w.
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        part[wave][r][lane] = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
+    __syncthreads();
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const float4 a = part[w][wave][lane];
+        v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+    }
+    total = ((red[1][0][n] + red[1][1][n]) + red[1][2][n]) + red[1][3][n];
+    const float inv = 1.0f / total;
+    bool bad = !(total > 0.0f);
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        v[d] *= inv;
+        bad |= !isfinite(v[d]);
+    }
+    const int t = 16 * f + n, c = head * kHeadDim + 16 * g + 4 * wave;
+    if constexpr (PLANES) {
+        store_planes4(out, t, positions, 0, c, v);
+    } else {
+#pragma unroll
+        for (int d = 0; d < 4; d++) rows[(size_t)t * kWidth + c + d] = v[d];
+    }
+    flag_nonfinite(status, bad);
 }
 
 // Orders one wave's LDS writes before its own later LDS reads: the hardware
@@ -75,21 +227,93 @@ __device__ inline void wave_lds_order() {
 }
 
 // A work-group computes 16 PT positions x 16 CT columns; its four waves take
-// a quarter of the input channels each. A wave stages one 32-channel block of
+// a quarter of the input channels each. A wave stages 32-channel blocks of
 // its tile's rows (taps - 1 more than positions) in its own part of LDS,
-// requests the next block and its weights, and then runs every tap from there:
+// requests the next ones and their weights, and then runs every tap from there:
 // tap j reads the same slots j rows further on, a 256-byte run per 16 lanes
 // either way.
-template <int TAPS, int PT, int CT>
-__global__ __launch_bounds__(256) void k_conv_planes(pgpu_plane_conv conv, pgpu_planes in,
-                                                     int positions, int phase, int past,
-                                                     float *__restrict__ rows, pgpu_planes out,
-                                                     int *status) {
+constexpr int taps_of(int epi) {
+    return epi == PGPU_PLANE_ROWS ? 2 : epi == PGPU_PLANE_ELU ? 7 : 1;
+}
+
+// 32-channel blocks a wave stages at once. A projection's one tap gives a
+// block too little work to hide the next one's latency (the MLP-out product,
+// 16 blocks a wave, took 11 us for one frame block by block); its small tiles
+// leave the registers and LDS for four. in.channels is a multiple of 512 then.
+constexpr int stage_blocks(int epi, int pt) { return taps_of(epi) == 1 ? 4 / pt : 1; }
+
+// Four results o (columns col .. col + 3 of position t) on their way out.
+// True if one is not finite.
+template <int EPI>
+__device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int positions, int phase,
+                                      int col, float *o) {
+    bool bad = false;
+    if constexpr (EPI == PGPU_PLANE_ROWS || EPI == PGPU_PLANE_ELU) {
+        const float4 b = *(const float4 *)(a.bias + col % a.cout);
+        o[0] = __fadd_rn(o[0], b.x);
+        o[1] = __fadd_rn(o[1], b.y);
+        o[2] = __fadd_rn(o[2], b.z);
+        o[3] = __fadd_rn(o[3], b.w);
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= !isfinite(o[r]);
+        if constexpr (EPI == PGPU_PLANE_ROWS) {
+            *(float4 *)(a.rows + (size_t)t * a.ncols + col) =
+                make_float4(o[0], o[1], o[2], o[3]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = elu1(o[r]);
+            store_planes4(a.planes, t, positions, phase, col, o);
+        }
+    } else if constexpr (EPI == PGPU_PLANE_GELU) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            o[r] = gelu_erf(o[r]);
+            bad |= !isfinite(o[r]);
+        }
+        store_planes4(a.planes, t, positions, phase, col, o);
+    } else if constexpr (EPI == PGPU_PLANE_GATED) {
+        float4 *at = (float4 *)(a.rows + (size_t)t * kWidth + col);
+        const float4 s = *at, k = *(const float4 *)(a.gate + col);
+        o[0] = __fadd_rn(s.x, __fmul_rn(k.x, o[0]));
+        o[1] = __fadd_rn(s.y, __fmul_rn(k.y, o[1]));
+        o[2] = __fadd_rn(s.z, __fmul_rn(k.z, o[2]));
+        o[3] = __fadd_rn(s.w, __fmul_rn(k.w, o[3]));
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= !isfinite(o[r]);
+        *at = make_float4(o[0], o[1], o[2], o[3]);
+        if (a.planes.data) store_planes4(a.planes, t, positions, phase, col, o);
+    } else {
+        const int part = col >> 9, c = col & 511;
+        const long long pos = a.first + t;
+        if (part < 2) {
+            const float4 cs = *(const float4 *)(a.rope + (size_t)pos * 64 + (c & 63));
+            const float v[4] = {o[0], o[1], o[2], o[3]};
+            o[0] = __fsub_rn(__fmul_rn(v[0], cs.x), __fmul_rn(v[1], cs.y));
+            o[1] = __fadd_rn(__fmul_rn(v[0], cs.y), __fmul_rn(v[1], cs.x));
+            o[2] = __fsub_rn(__fmul_rn(v[2], cs.z), __fmul_rn(v[3], cs.w));
+            o[3] = __fadd_rn(__fmul_rn(v[2], cs.w), __fmul_rn(v[3], cs.z));
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= !isfinite(o[r]);
+        float *dst = part == 0 ? a.rows + (size_t)t * kWidth
+                               : (part == 1 ? a.ring_k : a.ring_v) +
+                                     (size_t)(pos % a.ring) * kWidth;
+        *(float4 *)(dst + c) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+    return bad;
+}
+
+template <int EPI, int PT, int CT>
+__global__ __launch_bounds__(256) void k_plane_product(pgpu_plane_product a, pgpu_planes in,
+                                                       int positions, int phase, int past,
+                                                       int *status) {
+    constexpr int TAPS = taps_of(EPI), KS = stage_blocks(EPI, PT);
     constexpr int kRows = 16 * PT + TAPS - 1;
-    constexpr int kPieces = 12 * kRows;  // (term, octet of the block, row)
+    constexpr int kPieces = 12 * KS * kRows;  // (block, term, octet of the block, row)
     constexpr int kLoads = (kPieces + 63) / 64;
     constexpr int kStage = kLoads * 64;
     constexpr int kParts = 4 * PT * CT * 64;
+    static_assert(kLoads <= 32, "one bit of `zero` per load");
     __shared__ uint4 lds[4 * kStage > kParts ? 4 * kStage : kParts];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int t0 = blockIdx.x * 16 * PT, ct0 = blockIdx.y * CT;
@@ -102,14 +326,14 @@ __global__ __launch_bounds__(256) void k_conv_planes(pgpu_plane_conv conv, pgpu_
     for (int i = 0; i < kLoads; i++) {
         int piece = i * 64 + lane;
         piece = piece < kPieces ? piece : kPieces - 1;
-        const int to = piece / kRows;
+        const int to = piece / kRows, term = to % 12 >> 2;
         int r = t0 + piece % kRows - (TAPS - 1);
         r = r < positions ? r : positions - 1;
-        at[i] = ((to >> 2) * octets + 4 * cb0 + (to & 3)) * in.stride + slot_of(r, phase);
+        at[i] = (term * octets + 4 * (cb0 + to / 12) + (to & 3)) * in.stride + slot_of(r, phase);
         zero |= (uint32_t)(r < 0 && !past) << i;
     }
     const uint4 *src = (const uint4 *)in.data;
-    const int step = 4 * in.stride;
+    const int step = 4 * KS * in.stride;
     uint4 next[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; i++) next[i] = src[at[i]];
@@ -118,53 +342,58 @@ __global__ __launch_bounds__(256) void k_conv_planes(pgpu_plane_conv conv, pgpu_
     for (int p = 0; p < PT; p++)
 #pragma unroll
         for (int q = 0; q < CT; q++) acc[p][q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 *wsrc = (const bf16x8 *)conv.fragments + (size_t)ct0 * kbn * 64 + lane;
-    bf16x8 wnext[TAPS][CT];
+    const bf16x8 *wsrc = (const bf16x8 *)a.fragments + (size_t)ct0 * kbn * 64 + lane;
+    bf16x8 wnext[KS][TAPS][CT];
+    auto request_weights = [&](int cb) {
 #pragma unroll
-    for (int tap = 0; tap < TAPS; tap++)
+        for (int k = 0; k < KS; k++)
 #pragma unroll
-        for (int q = 0; q < CT; q++)
-            wnext[tap][q] = wsrc[(size_t)(q * kbn + tap * cbn + cb0) * 64];
-    for (int cb = cb0; cb < cb1; cb++) {
+            for (int tap = 0; tap < TAPS; tap++)
+#pragma unroll
+                for (int q = 0; q < CT; q++)
+                    wnext[k][tap][q] = wsrc[(size_t)(q * kbn + tap * cbn + cb + k) * 64];
+    };
+    request_weights(cb0);
+    for (int cb = cb0; cb < cb1; cb += KS) {
         wave_lds_order();
 #pragma unroll
         for (int i = 0; i < kLoads; i++)
             stage[i * 64 + lane] = (zero >> i) & 1 ? uint4{0, 0, 0, 0} : next[i];
-        bf16x8 wa[TAPS][CT];
+        bf16x8 wa[KS][TAPS][CT];
 #pragma unroll
-        for (int tap = 0; tap < TAPS; tap++)
+        for (int k = 0; k < KS; k++)
 #pragma unroll
-            for (int q = 0; q < CT; q++) wa[tap][q] = wnext[tap][q];
-        if (cb + 1 < cb1) {
+            for (int tap = 0; tap < TAPS; tap++)
+#pragma unroll
+                for (int q = 0; q < CT; q++) wa[k][tap][q] = wnext[k][tap][q];
+        if (cb + KS < cb1) {
 #pragma unroll
             for (int i = 0; i < kLoads; i++) {
                 at[i] += step;
                 next[i] = src[at[i]];
             }
-#pragma unroll
-            for (int tap = 0; tap < TAPS; tap++)
-#pragma unroll
-                for (int q = 0; q < CT; q++)
-                    wnext[tap][q] = wsrc[(size_t)(q * kbn + tap * cbn + cb + 1) * 64];
+            request_weights(cb + KS);
         }
         wave_lds_order();
 #pragma unroll
-        for (int tap = 0; tap < TAPS; tap++)
+        for (int k = 0; k < KS; k++)
 #pragma unroll
-            for (int term = 0; term < 3; term++) {
-                bf16x8 xs[PT];
+            for (int tap = 0; tap < TAPS; tap++)
 #pragma unroll
-                for (int p = 0; p < PT; p++)
-                    xs[p] = __builtin_bit_cast(
-                        bf16x8, stage[(term * 4 + (lane >> 4)) * kRows + p * 16 + (lane & 15) +
-                                      tap]);
+                for (int term = 0; term < 3; term++) {
+                    bf16x8 xs[PT];
 #pragma unroll
-                for (int p = 0; p < PT; p++)
+                    for (int p = 0; p < PT; p++)
+                        xs[p] = __builtin_bit_cast(
+                            bf16x8, stage[((k * 3 + term) * 4 + (lane >> 4)) * kRows + p * 16 +
+                                          (lane & 15) + tap]);
 #pragma unroll
-                    for (int q = 0; q < CT; q++)
-                        acc[p][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            wa[tap][q], xs[p], acc[p][q], 0, 0, 0);
-            }
+                    for (int p = 0; p < PT; p++)
+#pragma unroll
+                        for (int q = 0; q < CT; q++)
+                            acc[p][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                wa[k][tap][q], xs[p], acc[p][q], 0, 0, 0);
+                }
     }
     __syncthreads();
     f32x4 *part = (f32x4 *)lds;
@@ -185,18 +414,8 @@ __global__ __launch_bounds__(256) void k_conv_planes(pgpu_plane_conv conv, pgpu_
 #pragma unroll
             for (int r = 0; r < 4; r++) s[r] = __fadd_rn(s[r], o[r]);
         }
-        const float4 b = *(const float4 *)(conv.bias + col % conv.cout);
-        float o[4] = {__fadd_rn(s[0], b.x), __fadd_rn(s[1], b.y), __fadd_rn(s[2], b.z),
-                      __fadd_rn(s[3], b.w)};
-#pragma unroll
-        for (int r = 0; r < 4; r++) bad |= !isfinite(o[r]);
-        if constexpr (TAPS == 2) {
-            *(float4 *)(rows + (size_t)t * conv.ncols + col) = make_float4(o[0], o[1], o[2], o[3]);
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; r++) o[r] = elu1(o[r]);
-            store_planes4(out, t, positions, phase, col, o);
-        }
+        float o[4] = {s[0], s[1], s[2], s[3]};
+        bad |= plane_epilogue<EPI>(a, t, positions, phase, col, o);
     }
     flag_nonfinite(status, bad);
 }
@@ -432,33 +651,39 @@ bool planes_ok(const pgpu_planes *p, int positions) {
 
 bool pass_ok(pgpu_pass p) { return (p.phase == 0 || p.phase == 1) && (p.past == 0 || p.past == 1); }
 
-template <int TAPS, int PT, int CT>
-void launch_conv(hipStream_t st, const pgpu_plane_conv &c, const pgpu_planes &in, int positions,
-                 pgpu_pass pass, float *rows, const pgpu_planes &out, int *status) {
-    const dim3 grid((positions + 16 * PT - 1) / (16 * PT), c.ncols / (16 * CT));
-    hipLaunchKernelGGL((k_conv_planes<TAPS, PT, CT>), grid, dim3(256), 0, st, c, in, positions,
-                       pass.phase, pass.past, rows, out, status);
+template <int EPI, int PT, int CT>
+void launch_product(hipStream_t st, const pgpu_plane_product &a, const pgpu_planes &in,
+                    int positions, pgpu_pass pass, int *status) {
+    const dim3 grid((positions + 16 * PT - 1) / (16 * PT), a.ncols / (16 * CT));
+    hipLaunchKernelGGL((k_plane_product<EPI, PT, CT>), grid, dim3(256), 0, st, a, in, positions,
+                       pass.phase, pass.past, status);
 }
 
-// The largest tile that still leaves a work-group for (nearly) every CU:
-// larger tiles read each weight and row fewer times, smaller ones spread a
-// short pass over the chip.
-template <int TAPS>
-void launch_conv_tile(hipStream_t st, const pgpu_plane_conv &c, const pgpu_planes &in,
-                      int positions, pgpu_pass pass, float *rows, const pgpu_planes &out,
-                      int *status) {
+// Short passes are bound by latency, long ones by what the work-groups read
+// from L2: per reduction index a tile reads 2 bytes a column and 6 a position,
+// so tiles are wide in columns, and a larger one is taken as soon as it
+// leaves enough work-groups. conv0's seven taps of weights would not fit the
+// registers of a 64-column tile.
+template <int EPI>
+void launch_tile(hipStream_t st, const pgpu_plane_product &a, const pgpu_planes &in,
+                 int positions, pgpu_pass pass, int *status) {
     auto groups = [&](int pt, int ct) {
-        return (long)((positions + 16 * pt - 1) / (16 * pt)) * (c.ncols / (16 * ct));
+        return (long)((positions + 16 * pt - 1) / (16 * pt)) * (a.ncols / (16 * ct));
     };
-    constexpr long kFill = 224;
-    if (TAPS == 2 && groups(4, 4) >= kFill)
-        launch_conv<2, 4, 4>(st, c, in, positions, pass, rows, out, status);
-    else if (groups(4, 2) >= kFill)
-        launch_conv<TAPS, 4, 2>(st, c, in, positions, pass, rows, out, status);
-    else if (groups(2, 2) >= kFill)
-        launch_conv<TAPS, 2, 2>(st, c, in, positions, pass, rows, out, status);
-    else
-        launch_conv<TAPS, 1, 1>(st, c, in, positions, pass, rows, out, status);
+    if constexpr (EPI == PGPU_PLANE_ELU) {
+        if (groups(4, 2) >= 224)
+            return launch_product<EPI, 4, 2>(st, a, in, positions, pass, status);
+        if (groups(2, 2) >= 96)
+            return launch_product<EPI, 2, 2>(st, a, in, positions, pass, status);
+    } else {
+        if (groups(4, 4) >= 192)
+            return launch_product<EPI, 4, 4>(st, a, in, positions, pass, status);
+        if (groups(2, 4) >= 160)
+            return launch_product<EPI, 2, 4>(st, a, in, positions, pass, status);
+        if (groups(1, 4) >= 96)
+            return launch_product<EPI, 1, 4>(st, a, in, positions, pass, status);
+    }
+    launch_product<EPI, 1, 1>(st, a, in, positions, pass, status);
 }
 
 template <int C, int PT>
@@ -475,31 +700,92 @@ void launch_residual(hipStream_t st, const pgpu_residual_weights &w, const float
 
 using namespace pgpu;
 
-extern "C" int pgpu_pcm_rows_to_planes(void *stream, const float *rows, int positions,
-                                       const pgpu_planes *out, pgpu_pass pass) {
-    if (!rows || positions < 8 || !planes_ok(out, positions) || out->channels != kWidth ||
-        !pass_ok(pass))
-        return bad_arguments("pgpu_pcm_rows_to_planes");
-    hipLaunchKernelGGL(k_rows_to_planes, dim3((positions + 15) / 16, kWidth / 64), dim3(256), 0,
-                       (hipStream_t)stream, rows, positions, *out, pass.phase);
-    return launch_ok("pgpu_pcm_rows_to_planes");
+extern "C" int pgpu_pcm_layer_norm(void *stream, const float *rows, const float *weight,
+                                   const float *bias, float epsilon, int positions,
+                                   const pgpu_planes *out, int *status) {
+    if (!rows || !weight || !bias || !(epsilon > 0.0f) || positions <= 0 ||
+        !planes_ok(out, positions) || out->channels != kWidth || !status)
+        return bad_arguments("pgpu_pcm_layer_norm");
+    hipLaunchKernelGGL(k_ln_planes, dim3((positions + 7) / 8), dim3(256), 0, (hipStream_t)stream,
+                       rows, weight, bias, epsilon, positions, *out, status);
+    return launch_ok("pgpu_pcm_layer_norm");
 }
 
-extern "C" int pgpu_pcm_conv(void *stream, const pgpu_plane_conv *c, const pgpu_planes *in,
-                             int positions, pgpu_pass pass, float *rows, const pgpu_planes *planes,
-                             int *status) {
-    if (!c || !c->fragments || !c->bias || positions < 8 || !planes_ok(in, positions) ||
-        in->channels % 128 || c->ncols <= 0 || c->ncols % 64 || c->cout <= 0 || c->cout % 64 ||
-        !pass_ok(pass) || !status || (c->taps != 2 && c->taps != 7) || (c->taps == 2 && !rows) ||
-        (c->taps == 7 && (!planes_ok(planes, positions) || planes->channels != c->ncols)) ||
-        (long)(positions + 15) / 16 * (c->ncols / 16) > 0x7fffffL)
-        return bad_arguments("pgpu_pcm_conv");
+static bool attention_ok(const float *q, int rows, long long first, const float *ring_k,
+                         const float *ring_v, int ring, int context, const int *status) {
+    return q && rows > 0 && rows % 16 == 0 && rows <= 65535 && first >= 0 && ring_k && ring_v &&
+           context > 0 && context <= 256 && ring >= rows + context - 1 && status;
+}
+
+extern "C" int pgpu_pcm_attention(void *stream, const float *q, int rows, long long first,
+                                  const float *ring_k, const float *ring_v, int ring, int context,
+                                  const pgpu_planes *out, int *status) {
+    if (!attention_ok(q, rows, first, ring_k, ring_v, ring, context, status) ||
+        !planes_ok(out, rows) || out->channels != kWidth)
+        return bad_arguments("pgpu_pcm_attention");
+    hipLaunchKernelGGL(k_window_attention<true>, dim3(rows / 16, kHeads), dim3(256), 0,
+                       (hipStream_t)stream, q, kWidth, first, ring_k, ring_v, ring, context,
+                       nullptr, *out, rows, status);
+    return launch_ok("pgpu_pcm_attention");
+}
+
+extern "C" int pgpu_mimi_attention(void *stream, const float *qkv, int rows, long long first,
+                                   const float *ring_k, const float *ring_v, int ring,
+                                   int context, float *out, int *status) {
+    if (!attention_ok(qkv, rows, first, ring_k, ring_v, ring, context, status) || !out)
+        return bad_arguments("pgpu_mimi_attention");
+    hipLaunchKernelGGL(k_window_attention<false>, dim3(rows / 16, kHeads), dim3(256), 0,
+                       (hipStream_t)stream, qkv, 3 * kWidth, first, ring_k, ring_v, ring, context,
+                       out, pgpu_planes{}, rows, status);
+    return launch_ok("pgpu_mimi_attention");
+}
+
+static bool product_ok(const pgpu_plane_product *a, const pgpu_planes *in, int positions) {
+    if (!a || !a->fragments || positions < 8 || !planes_ok(in, positions) || in->channels % 128 ||
+        a->ncols <= 0 || a->ncols % 64 ||
+        (long)(positions + 15) / 16 * (a->ncols / 16) > 0x7fffffL)
+        return false;
+    const bool planes = planes_ok(&a->planes, positions) && a->planes.channels == a->ncols;
+    switch (a->epilogue) {
+    case PGPU_PLANE_ROWS:
+        return a->rows && a->bias && a->cout > 0 && a->cout % 64 == 0;
+    case PGPU_PLANE_ELU:
+        return planes && a->bias && a->cout > 0 && a->cout % 64 == 0;
+    case PGPU_PLANE_GELU:
+        return planes && in->channels % 512 == 0;
+    case PGPU_PLANE_GATED:
+        return a->rows && a->gate && a->ncols == kWidth && (!a->planes.data || planes) &&
+               in->channels % 512 == 0;
+    case PGPU_PLANE_QKV:
+        return a->rows && in->channels % 512 == 0 && a->ncols == 3 * kWidth && a->rope && a->first >= 0 &&
+               a->first + positions <= a->rope_positions && a->ring_k && a->ring_v &&
+               a->ring >= positions;
+    }
+    return false;
+}
+
+extern "C" int pgpu_pcm_product(void *stream, const pgpu_plane_product *a, const pgpu_planes *in,
+                                int positions, pgpu_pass pass, int *status) {
+    if (!product_ok(a, in, positions) || !pass_ok(pass) || !status)
+        return bad_arguments("pgpu_pcm_product");
     hipStream_t st = (hipStream_t)stream;
-    if (c->taps == 2)
-        launch_conv_tile<2>(st, *c, *in, positions, pass, rows, pgpu_planes{}, status);
-    else
-        launch_conv_tile<7>(st, *c, *in, positions, pass, nullptr, *planes, status);
-    return launch_ok("pgpu_pcm_conv");
+    switch (a->epilogue) {
+    case PGPU_PLANE_ROWS:
+        launch_tile<PGPU_PLANE_ROWS>(st, *a, *in, positions, pass, status);
+        break;
+    case PGPU_PLANE_ELU:
+        launch_tile<PGPU_PLANE_ELU>(st, *a, *in, positions, pass, status);
+        break;
+    case PGPU_PLANE_GELU:
+        launch_tile<PGPU_PLANE_GELU>(st, *a, *in, positions, pass, status);
+        break;
+    case PGPU_PLANE_GATED:
+        launch_tile<PGPU_PLANE_GATED>(st, *a, *in, positions, pass, status);
+        break;
+    default:
+        launch_tile<PGPU_PLANE_QKV>(st, *a, *in, positions, pass, status);
+    }
+    return launch_ok("pgpu_pcm_product");
 }
 
 extern "C" int pgpu_pcm_residual(void *stream, const pgpu_residual_weights *w, int channels,

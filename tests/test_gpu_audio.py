@@ -147,6 +147,38 @@ def test_mimi_random_weights_ring_wrap_against_oracle(lib, pkg, oracle, oracle_m
     m.close()
 
 
+@pytest.mark.parametrize("first,frames,context,ring", [
+    (0, 2, 1, 32), (0, 3, 250, 304), (1008, 3, 250, 1024), (4096, 2, 256, 287)])
+def test_mimi_attention_windows(lib, pkg, first, frames, context, ring):
+    """The window attention against float64 softmax: one key, a window that
+    starts inside the first frames, one that wraps the ring (an odd-sized ring
+    among them) and the longest window. fp32 sums over at most 271 keys: 1e-5
+    of the largest output."""
+    rows = 16 * frames
+    rng = np.random.default_rng(first + context)
+    qkv = rng.standard_normal((rows, 1536)).astype(np.float32)
+    kv = rng.standard_normal((2, ring, 512)).astype(np.float32)
+    bufs = [pkg.DeviceBuffer(lib, a.nbytes) for a in (qkv, kv[0], kv[1], qkv[:, :512])]
+    status = pkg.DeviceBuffer(lib, 4)
+    for b, a in zip(bufs + [status], (qkv, kv[0], kv[1], np.zeros((rows, 512), np.float32),
+                                      np.zeros(1, np.int32))):
+        b.upload(a)
+    assert lib.pgpu_mimi_attention(None, bufs[0].ptr, rows, first, bufs[1].ptr, bufs[2].ptr, ring,
+                                   context, bufs[3].ptr, status.ptr) == 1
+    got = bufs[3].download((rows, 512), np.float32)
+    assert status.download((1,), np.int32)[0] == 0
+    exp = np.zeros((rows, 512))
+    for r in range(rows):
+        p = first + r
+        at = np.arange(max(0, p - context + 1), p + 1) % ring
+        for h in range(8):
+            d = slice(64 * h, 64 * h + 64)
+            score = kv[0][at, d].astype(np.float64) @ qkv[r, d].astype(np.float64) / 8
+            e = np.exp(score - score.max())
+            exp[r, d] = e @ kv[1][at, d].astype(np.float64) / e.sum()
+    assert normwise(got, exp) <= 1e-5
+
+
 def test_mimi_rejects_bad_requests(lib, pkg):
     views = pkg.Views()
     model = mimi_model(lib, pkg, views, mimi_identity_model())
