@@ -16,6 +16,7 @@
 // stored [input channel][tap][output channel] so that a wave's loads are
 // contiguous.
 #include "pgpu_common.hpp"
+#include "pgpu_pcm.h"
 #include "phonon_gpu.h"
 
 namespace pgpu {
@@ -26,21 +27,50 @@ constexpr int kMimiRows = 16;  // feature rows per latent frame
 // Projection (512 x 32) and depthwise upsample of every latent frame:
 // hidden[16 f + o][c] = prev[c] * k[c][16 + o] + cur[c] * k[c][o], where
 // cur is frame f's projection and prev frame f - 1's (the state's
-// `previous` for f = 0). The last frame's projection becomes `previous`.
+// `previous` for f = 0, zero when nothing came before). The last frame's
+// projection becomes `previous`: only frame 0's work-groups read it, and the
+// same threads replace it. The latents go through LDS in one load, since they
+// may lie in host memory. Work-groups past the frames put the positions that
+// a request kept of its convolutions' inputs back into their slots 0 .. 7.
 __global__ __launch_bounds__(256) void k_mimi_input(const float *__restrict__ latents, int frames,
                                                     const float *__restrict__ proj,
                                                     const float *__restrict__ upk,
-                                                    float *__restrict__ previous,
-                                                    float *__restrict__ hidden, int *status) {
+                                                    float *__restrict__ previous, int past,
+                                                    pgpu_kept keep, float *__restrict__ hidden,
+                                                    int *status) {
+    __shared__ float lat[3][32];  // frames f - 1, f and (for f = 0) the last
+    if ((int)blockIdx.x >= frames) {  // uniform
+        int i = (((int)blockIdx.x - frames) * 2 + blockIdx.y) * 256 + threadIdx.x;
+        if (i >= PGPU_KEPT_SLOTS) return;
+        const uint4 v = ((const uint4 *)keep.kept)[i];
+        for (int p = 0; p < PGPU_KEPT_PLANES; p++) {
+            const int count = 3 * keep.in[p].channels;
+            if (i < count) {
+                ((uint4 *)keep.in[p].data)[(size_t)(i >> 3) * keep.in[p].stride + (i & 7)] = v;
+                return;
+            }
+            i -= count;
+        }
+        return;
+    }
     const int f = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
-    auto project = [&](int frame) {
+    if (threadIdx.x < 96) {
+        const int j = threadIdx.x >> 5;
+        const int frame = j == 0 ? (f > 0 ? f - 1 : 0) : j == 1 ? f : frames - 1;
+        lat[j][threadIdx.x & 31] = latents[frame * 32 + (threadIdx.x & 31)];
+    }
+    float w[32];
+#pragma unroll
+    for (int i = 0; i < 32; i++) w[i] = proj[c * 32 + i];
+    __syncthreads();
+    auto project = [&](int j) {
         float dot = 0.0f;
-#pragma unroll 8
-        for (int i = 0; i < 32; i++) dot = dot + proj[c * 32 + i] * latents[frame * 32 + i];
+#pragma unroll
+        for (int i = 0; i < 32; i++) dot = dot + w[i] * lat[j][i];
         return dot;
     };
-    const float cur = project(f);
-    const float prev = f == 0 ? previous[c] : project(f - 1);
+    const float cur = project(1);
+    const float prev = f > 0 ? project(0) : past ? previous[c] : 0.0f;
     bool bad = !isfinite(cur) || !isfinite(prev);
 #pragma unroll
     for (int o = 0; o < kMimiRows; o++) {
@@ -51,8 +81,7 @@ __global__ __launch_bounds__(256) void k_mimi_input(const float *__restrict__ la
         hidden[((size_t)f * kMimiRows + o) * kWidth + c] = v;
     }
     flag_nonfinite(status, bad);
-    // Only frame 0's work-groups read `previous`; the same threads replace it.
-    if (f == 0) previous[c] = frames > 1 ? project(frames - 1) : cur;
+    if (f == 0) previous[c] = project(2);
 }
 
 // RoPE of q and k of every row (position first + r), then k and v into the
@@ -332,16 +361,25 @@ extern "C" int pgpu_upsample_frame(void *stream, const float *kernel, const floa
     return launch_ok("pgpu_upsample_frame");
 }
 
-extern "C" int pgpu_mimi_input(void *stream, const float *latents, int frames,
-                               const float *projection, const float *upsample, float *previous,
-                               float *hidden, int *status) {
+extern "C" int pgpu_pcm_input(void *stream, const float *latents, int frames,
+                              const float *projection, const float *upsample, float *previous,
+                              int past, const pgpu_kept *keep, float *hidden, int *status) {
     if (!latents || frames <= 0 || frames > 65535 || !projection || !upsample || !previous ||
         !hidden || !status)
         return bad_arguments("pgpu_mimi_input");
-    hipLaunchKernelGGL(k_mimi_input, dim3(frames, kWidth / 256), dim3(256), 0,
+    static_assert(kWidth / 256 == 2, "two work-groups per frame");
+    const int restore = past && keep ? (PGPU_KEPT_SLOTS + 511) / 512 : 0;
+    hipLaunchKernelGGL(k_mimi_input, dim3(frames + restore, 2), dim3(256), 0,
                        (hipStream_t)stream, latents, frames, projection, upsample, previous,
-                       hidden, status);
+                       past, restore ? *keep : pgpu_kept{}, hidden, status);
     return launch_ok("pgpu_mimi_input");
+}
+
+extern "C" int pgpu_mimi_input(void *stream, const float *latents, int frames,
+                               const float *projection, const float *upsample, float *previous,
+                               float *hidden, int *status) {
+    return pgpu_pcm_input(stream, latents, frames, projection, upsample, previous, 1, nullptr,
+                          hidden, status);
 }
 
 extern "C" int pgpu_mimi_rope_store(void *stream, float *qkv, int rows, long long first,

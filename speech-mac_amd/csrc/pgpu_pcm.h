@@ -5,11 +5,8 @@
  *
  * A "planes" buffer holds a convolution's input as the three exact bf16
  * terms of each value (hi + mid + lo): [3][channels / 8][stride][8] bf16, a
- * 16-byte slot per (term, 8 channels, position). Slot 16 + r is the pass's
- * position r; the 8 positions before the pass are slots 8 phase .. 8 phase
- * + 7, where the previous pass's producer put its last 8. phase alternates
- * from pass to pass, so a producer never writes what its pass's consumer
- * still reads. */
+ * 16-byte slot per (term, 8 channels, position). Slot 8 + r is position r of
+ * the pass, so that the 8 positions before it are slots 0 .. 7. */
 #ifndef PGPU_PCM_H
 #define PGPU_PCM_H
 
@@ -23,14 +20,37 @@ extern "C" {
 typedef struct {
     uint16_t *data;
     int channels; /* a multiple of 32 */
-    int stride;   /* slots: 16 + the largest pass's positions */
+    int stride;   /* slots: 8 + the largest pass's positions */
 } pgpu_planes;
 
 /* Where a pass stands in its request. */
 typedef struct {
-    int phase; /* 0 or 1, alternating */
+    int phase; /* 0 or 1, alternating: which half of a residual pair's history */
     int past;  /* 0: the request's first pass (what came before is zero) */
 } pgpu_pass;
+
+/* What a request keeps of its convolutions' inputs between passes (the planes
+ * themselves are only borrowed for a call): the last 8 positions of each,
+ * [PGPU_KEPT_SLOTS] slots. */
+enum { PGPU_KEPT_PLANES = 4, PGPU_KEPT_SLOTS = 8 * 3 * (512 + 512 + 256 + 128) / 8 };
+typedef struct {
+    pgpu_planes in[PGPU_KEPT_PLANES]; /* channels 512, 512, 256, 128 */
+    int positions[PGPU_KEPT_PLANES];  /* of the pass */
+    uint16_t *kept;
+} pgpu_kept;
+
+/* The first launch of a pass: pgpu_mimi_input (pgpu_audio.hip), whose
+ * `latents` may be pinned host memory and whose `previous` is taken as zero
+ * when past is 0, and, when it is 1 and keep given, the kept positions put
+ * back before the pass's own. */
+int pgpu_pcm_input(void *stream, const float *latents, int frames, const float *projection,
+                   const float *upsample, float *previous, int past, const pgpu_kept *keep,
+                   float *hidden, int *status);
+
+/* The last one: the pass's last positions kept, and *seen = *status (seen:
+ * pinned host memory); then the wait for an event recorded after it. */
+int pgpu_pcm_keep(void *stream, const pgpu_kept *keep, const int *status, int *seen);
+int pgpu_pcm_wait(void *event);
 
 /* LayerNorm of rows [positions][512] -> planes. */
 int pgpu_pcm_layer_norm(void *stream, const float *rows, const float *weight, const float *bias,
@@ -72,7 +92,7 @@ int pgpu_pcm_attention(void *stream, const float *q, int rows, long long first,
 /* A residual pair over x [positions][channels], channels 256, 128 or 64:
  * v = x + conv1(ELU(conv3(ELU(x)))). channels 256 and 128: ELU(v) into
  * `planes`. channels 64: the output convolution (3 taps, 64 -> 1) of ELU(v)
- * into pcm [positions]. history [2][4][channels] holds x's rows before the
+ * into pcm [positions] (device or pinned host memory). history [2][4][channels] holds x's rows before the
  * pass (by phase) and receives its last four. positions >= 8. */
 typedef struct {
     const uint16_t *conv3, *conv1, *last; /* fragments; last: channels 64 only */

@@ -27,21 +27,15 @@
 namespace pgpu {
 namespace {
 
-constexpr int kSlots = 16;  // slots before a planes buffer's own positions
+constexpr int kSlots = 8;  // slots before a planes buffer's own positions
 
 __device__ inline float elu1(float v) { return v <= 0.0f ? expf(v) - 1.0f : v; }
 
 __device__ inline uint32_t pack16(uint16_t a, uint16_t b) { return a | (uint32_t)b << 16; }
 
-// Slot of position r >= -8 of the pass.
-__device__ inline int slot_of(int r, int phase) {
-    return r < 0 ? 8 * phase + 8 + r : kSlots + r;
-}
-
 // Four consecutive channels (c % 4 == 0) of position t as the planes' three
-// terms; the last 8 positions also where the next pass finds its past.
-__device__ inline void store_planes4(const pgpu_planes &out, int t, int positions, int phase,
-                                     int c, const float *v) {
+// terms.
+__device__ inline void store_planes4(const pgpu_planes &out, int t, int c, const float *v) {
     uint16_t h[4], m[4], l[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) split3(v[i], h[i], m[i], l[i]);
@@ -50,13 +44,9 @@ __device__ inline void store_planes4(const pgpu_planes &out, int t, int position
                            {pack16(l[0], l[1]), pack16(l[2], l[3])}};
     const int octets = out.channels >> 3;
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        uint2 *p = (uint2 *)out.data +
-                   ((size_t)(i * octets + (c >> 3)) * out.stride) * 2 + ((c >> 2) & 1);
-        p[(size_t)(kSlots + t) * 2] = term[i];
-        if (t >= positions - 8)
-            p[(size_t)slot_of(t - positions, 1 - phase) * 2] = term[i];
-    }
+    for (int i = 0; i < 3; i++)
+        ((uint2 *)out.data)[((size_t)(i * octets + (c >> 3)) * out.stride + kSlots + t) * 2 +
+                            ((c >> 2) & 1)] = term[i];
 }
 
 // A wave normalises two rows with the decode step's LayerNorm arithmetic;
@@ -113,7 +103,7 @@ template <bool PLANES>
 __global__ __launch_bounds__(256) void k_window_attention(
     const float *__restrict__ q, int ld_q, long long first, const float *__restrict__ ring_k,
     const float *__restrict__ ring_v, int ring, int context, float *__restrict__ rows,
-    pgpu_planes out, int positions, int *status) {
+    pgpu_planes out, int *status) {
     __shared__ float red[2][4][16];
     __shared__ float4 part[4][4][64];
     const int f = blockIdx.x, head = blockIdx.y;
@@ -210,7 +200,7 @@ __global__ __launch_bounds__(256) void k_window_attention(
     }
     const int t = 16 * f + n, c = head * kHeadDim + 16 * g + 4 * wave;
     if constexpr (PLANES) {
-        store_planes4(out, t, positions, 0, c, v);
+        store_planes4(out, t, c, v);
     } else {
 #pragma unroll
         for (int d = 0; d < 4; d++) rows[(size_t)t * kWidth + c + d] = v[d];
@@ -245,8 +235,7 @@ constexpr int stage_blocks(int epi, int pt) { return taps_of(epi) == 1 ? 4 / pt 
 // Four results o (columns col .. col + 3 of position t) on their way out.
 // True if one is not finite.
 template <int EPI>
-__device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int positions, int phase,
-                                      int col, float *o) {
+__device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int col, float *o) {
     bool bad = false;
     if constexpr (EPI == PGPU_PLANE_ROWS || EPI == PGPU_PLANE_ELU) {
         const float4 b = *(const float4 *)(a.bias + col % a.cout);
@@ -262,7 +251,7 @@ __device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int po
         } else {
 #pragma unroll
             for (int r = 0; r < 4; r++) o[r] = elu1(o[r]);
-            store_planes4(a.planes, t, positions, phase, col, o);
+            store_planes4(a.planes, t, col, o);
         }
     } else if constexpr (EPI == PGPU_PLANE_GELU) {
 #pragma unroll
@@ -270,7 +259,7 @@ __device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int po
             o[r] = gelu_erf(o[r]);
             bad |= !isfinite(o[r]);
         }
-        store_planes4(a.planes, t, positions, phase, col, o);
+        store_planes4(a.planes, t, col, o);
     } else if constexpr (EPI == PGPU_PLANE_GATED) {
         float4 *at = (float4 *)(a.rows + (size_t)t * kWidth + col);
         const float4 s = *at, k = *(const float4 *)(a.gate + col);
@@ -281,7 +270,7 @@ __device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int po
 #pragma unroll
         for (int r = 0; r < 4; r++) bad |= !isfinite(o[r]);
         *at = make_float4(o[0], o[1], o[2], o[3]);
-        if (a.planes.data) store_planes4(a.planes, t, positions, phase, col, o);
+        if (a.planes.data) store_planes4(a.planes, t, col, o);
     } else {
         const int part = col >> 9, c = col & 511;
         const long long pos = a.first + t;
@@ -305,8 +294,7 @@ __device__ inline bool plane_epilogue(const pgpu_plane_product &a, int t, int po
 
 template <int EPI, int PT, int CT>
 __global__ __launch_bounds__(256) void k_plane_product(pgpu_plane_product a, pgpu_planes in,
-                                                       int positions, int phase, int past,
-                                                       int *status) {
+                                                       int positions, int past, int *status) {
     constexpr int TAPS = taps_of(EPI), KS = stage_blocks(EPI, PT);
     constexpr int kRows = 16 * PT + TAPS - 1;
     constexpr int kPieces = 12 * KS * kRows;  // (block, term, octet of the block, row)
@@ -329,7 +317,7 @@ __global__ __launch_bounds__(256) void k_plane_product(pgpu_plane_product a, pgp
         const int to = piece / kRows, term = to % 12 >> 2;
         int r = t0 + piece % kRows - (TAPS - 1);
         r = r < positions ? r : positions - 1;
-        at[i] = (term * octets + 4 * (cb0 + to / 12) + (to & 3)) * in.stride + slot_of(r, phase);
+        at[i] = (term * octets + 4 * (cb0 + to / 12) + (to & 3)) * in.stride + kSlots + r;
         zero |= (uint32_t)(r < 0 && !past) << i;
     }
     const uint4 *src = (const uint4 *)in.data;
@@ -415,7 +403,7 @@ __global__ __launch_bounds__(256) void k_plane_product(pgpu_plane_product a, pgp
             for (int r = 0; r < 4; r++) s[r] = __fadd_rn(s[r], o[r]);
         }
         float o[4] = {s[0], s[1], s[2], s[3]};
-        bad |= plane_epilogue<EPI>(a, t, positions, phase, col, o);
+        bad |= plane_epilogue<EPI>(a, t, col, o);
     }
     flag_nonfinite(status, bad);
 }
@@ -609,7 +597,7 @@ __global__ __launch_bounds__(64 * kResWaves) void k_residual(
                 if constexpr (kLast)
                     *(float4 *)(es + j * kE + c) = make_float4(o[0], o[1], o[2], o[3]);
                 else if (live)
-                    store_planes4(out, t, positions, phase, c, o);
+                    store_planes4(out, t, c, o);
             }
     }
     if constexpr (kLast) {
@@ -643,6 +631,26 @@ __global__ __launch_bounds__(64 * kResWaves) void k_residual(
     flag_nonfinite(status, bad);
 }
 
+// The last 8 positions of each convolution's input, and the status word.
+__global__ __launch_bounds__(256) void k_keep(pgpu_kept keep, const int *__restrict__ status,
+                                              int *__restrict__ seen) {
+    int i = blockIdx.x * 256 + threadIdx.x;
+    if (i == 0) *seen = *status;
+    if (i >= PGPU_KEPT_SLOTS) return;
+    uint4 *dst = (uint4 *)keep.kept + i;
+#pragma unroll
+    for (int p = 0; p < PGPU_KEPT_PLANES; p++) {
+        const pgpu_planes &in = keep.in[p];
+        const int count = 3 * in.channels;  // slots: 8 of each (term, octet)
+        if (i < count) {
+            *dst = ((const uint4 *)in.data)[(size_t)(i >> 3) * in.stride + keep.positions[p] +
+                                            (i & 7)];
+            return;
+        }
+        i -= count;
+    }
+}
+
 bool planes_ok(const pgpu_planes *p, int positions) {
     return p && p->data && p->channels > 0 && p->channels % 32 == 0 &&
            p->stride >= kSlots + positions &&
@@ -656,7 +664,7 @@ void launch_product(hipStream_t st, const pgpu_plane_product &a, const pgpu_plan
                     int positions, pgpu_pass pass, int *status) {
     const dim3 grid((positions + 16 * PT - 1) / (16 * PT), a.ncols / (16 * CT));
     hipLaunchKernelGGL((k_plane_product<EPI, PT, CT>), grid, dim3(256), 0, st, a, in, positions,
-                       pass.phase, pass.past, status);
+                       pass.past, status);
 }
 
 // Short passes are bound by latency, long ones by what the work-groups read
@@ -700,6 +708,24 @@ void launch_residual(hipStream_t st, const pgpu_residual_weights &w, const float
 
 using namespace pgpu;
 
+extern "C" int pgpu_pcm_keep(void *stream, const pgpu_kept *keep, const int *status, int *seen) {
+    constexpr int channels[PGPU_KEPT_PLANES] = {512, 512, 256, 128};
+    bool ok = keep && keep->kept && status && seen;
+    for (int p = 0; ok && p < PGPU_KEPT_PLANES; p++)
+        ok = keep->positions[p] >= 8 && planes_ok(&keep->in[p], keep->positions[p]) &&
+             keep->in[p].channels == channels[p];
+    if (!ok) return bad_arguments("pgpu_pcm_keep");
+    hipLaunchKernelGGL(k_keep, dim3((PGPU_KEPT_SLOTS + 255) / 256), dim3(256), 0,
+                       (hipStream_t)stream, *keep, status, seen);
+    return launch_ok("pgpu_pcm_keep");
+}
+
+extern "C" int pgpu_pcm_wait(void *event) {
+    if (hipEventSynchronize((hipEvent_t)event) == hipSuccess) return 1;
+    pgpu_record_error("pgpu_pcm_wait: hipEventSynchronize failed");
+    return 0;
+}
+
 extern "C" int pgpu_pcm_layer_norm(void *stream, const float *rows, const float *weight,
                                    const float *bias, float epsilon, int positions,
                                    const pgpu_planes *out, int *status) {
@@ -725,7 +751,7 @@ extern "C" int pgpu_pcm_attention(void *stream, const float *q, int rows, long l
         return bad_arguments("pgpu_pcm_attention");
     hipLaunchKernelGGL(k_window_attention<true>, dim3(rows / 16, kHeads), dim3(256), 0,
                        (hipStream_t)stream, q, kWidth, first, ring_k, ring_v, ring, context,
-                       nullptr, *out, rows, status);
+                       nullptr, *out, status);
     return launch_ok("pgpu_pcm_attention");
 }
 
@@ -736,7 +762,7 @@ extern "C" int pgpu_mimi_attention(void *stream, const float *qkv, int rows, lon
         return bad_arguments("pgpu_mimi_attention");
     hipLaunchKernelGGL(k_window_attention<false>, dim3(rows / 16, kHeads), dim3(256), 0,
                        (hipStream_t)stream, qkv, 3 * kWidth, first, ring_k, ring_v, ring, context,
-                       out, pgpu_planes{}, rows, status);
+                       out, pgpu_planes{}, status);
     return launch_ok("pgpu_mimi_attention");
 }
 

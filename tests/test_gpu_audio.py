@@ -421,12 +421,13 @@ def test_pcm_random_weights_against_oracle(lib, pkg, oracle, oracle_mod):
     p.close()
 
 
-@pytest.mark.parametrize("counts", [(1,) * 9, (2, 3, 4), (7, 2), (12, 20, 32), (33, 31)])
+@pytest.mark.parametrize("counts", [(1,) * 9, (2, 3, 4), (7, 2), (12, 20, 32), (64, 1), (65,),
+                                    (9, 140)])
 def test_pcm_tile_shapes_and_passes(lib, pkg, oracle, oracle_mod, counts):
     """Calls whose passes take each tile shape of the convolutions (from one
-    frame's 16 positions to a full pass, with remainders), and requests after a
-    reset: the bits of one frame at a time, whose first frames are the oracle's.
-    The state first runs another request, whose rows a new one must not see."""
+    frame's 16 positions to a full pass, with remainders), calls of two and three
+    passes, the ring's wrap (past 128 frames) and requests after a reset: the bits
+    of one frame at a time, whose first frames are the oracle's. The state first runs another request, whose rows a new one must not see."""
     mimi_w, convs = random_mimi(911), random_pcm_convs(912)
     frames = sum(counts)
     x = np.random.default_rng(913).standard_normal((frames, 32)).astype(np.float32)
@@ -455,6 +456,35 @@ def test_pcm_tile_shapes_and_passes(lib, pkg, oracle, oracle_mod, counts):
     om.close()
     assert ok and normwise(single[:known * 1920], exp) <= TOL
     p.close()
+
+
+def test_pcm_calls_from_several_threads(lib, pkg):
+    """Four states, each in a thread of its own, more calls at once than the
+    library keeps staging memory for: every request has the bits of the same
+    request alone."""
+    import threading
+    views = pkg.Views()
+    mimi_w, convs = random_mimi(921), random_pcm_convs(922)
+    states = [Pcm(lib, pkg, views, mimi_w, convs) for _ in range(4)]
+    rng = np.random.default_rng(923)
+    x = [rng.standard_normal((n, 32)).astype(np.float32) for n in (70, 3, 33, 1)]
+    alone = [p.process(a) for p, a in zip(states, x)]
+    got = [None] * 4
+
+    def request(i):
+        for _ in range(5):
+            lib.phonon_pcm_state_reset(states[i].h)
+            got[i] = states[i].process(x[i])
+
+    threads = [threading.Thread(target=request, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (ok, raw, _), (ok1, raw1, _) in zip(got, alone):
+        assert ok == 1 and ok1 == 1 and np.array_equal(raw, raw1)
+    for p in states:
+        p.close()
 
 
 def test_pcm_rejects_bad_requests(lib, pkg):
