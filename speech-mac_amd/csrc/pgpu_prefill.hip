@@ -39,6 +39,7 @@
 // step's in summation order only (fp32 throughout).
 #include "pgpu_attention.hpp"
 #include "pgpu_gemm.hpp"
+#include "pgpu_prefill.h"
 #include "phonon_gpu.h"
 
 namespace pgpu {
@@ -470,6 +471,148 @@ __global__ __launch_bounds__(kTaskThreads) void k_prefill_gemm(GemmArgs a, int r
             const int row0 = (rt0 + wr * RW + r) * 16 + (lane >> 4) * 4;
             bad |= epilogue<EPI, FORMAT>(a, ep[r][p], tot[r][p], s, row0, s < a.streams);
         }
+    flag_nonfinite(a.status, bad);
+}
+
+// ---------------------------------------------------------------------------
+// Projection of up to some thousand positions (fast prefill). k_prefill_gemm
+// shares its operands among eight waves through LDS, which costs a barrier
+// and a copy wait per stage: with too few work-groups to overlap them, a
+// 611-position MLP-out product took 26 us (its 64 column blocks one after
+// the other) on 40 work-groups. Here each wave takes one of the summation
+// chains (8 column blocks: K = 2048 has eight, K = 512 two for each of four
+// groups of row tiles) and loads its own operands, which the split fragments
+// and the weights hold in operand order, straight into registers: the only
+// barrier is the one before the chains are added, in order, so the outputs
+// have k_prefill_gemm's bits. A tile's operands then come from L2 once per
+// work-group that uses them.
+template <int EPI, bool SCALED, int CHAINS, int RW, int PW, int FORMAT>
+__global__ __launch_bounds__(kTaskThreads) void k_prefill_split(GemmArgs a, int row_groups,
+                                                                int pos_groups) {
+    constexpr int TERMS = split_records(FORMAT), kWr = kTaskWaves / CHAINS;
+    constexpr bool F16 = FORMAT == kF16Pair;
+    constexpr int kTiles = RW * PW, kbn = CHAINS * kChain;
+    __shared__ f32x4 part[kTaskWaves * kTiles * 64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int chain = wave / kWr, wr = wave % kWr;
+    // Position groups over the XCDs, as in k_prefill_gemm.
+    int row_group, pos_group;
+    if (pos_groups % 8 == 0) {
+        const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+        pos_group = xcd + 8 * (local / row_groups);
+        row_group = local % row_groups;
+    } else {
+        pos_group = blockIdx.x / row_groups;
+        row_group = blockIdx.x % row_groups;
+    }
+    const int pt0 = pos_group * PW, rt0 = (row_group * kWr + wr) * RW;
+    const int last_tile = (a.streams - 1) >> 4, kb0 = chain * kChain;
+    const bf16x8 *xsrc[PW], *wsrc[RW];
+    const float4 *ssrc[RW];
+#pragma unroll
+    for (int p = 0; p < PW; p++)
+        xsrc[p] = (const bf16x8 *)(a.xs + ((size_t)min(pt0 + p, last_tile) * kbn + kb0) * 1536);
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        wsrc[r] = (const bf16x8 *)a.w + ((size_t)(rt0 + r) * kbn + kb0) * 64;
+        if constexpr (SCALED)
+            ssrc[r] = (const float4 *)(a.wscale_f + ((size_t)(rt0 + r) * kbn + kb0) * 16);
+    }
+    f32x4 acc[RW][PW];
+#pragma unroll
+    for (int r = 0; r < RW; r++)
+#pragma unroll
+        for (int p = 0; p < PW; p++) acc[r][p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // kDepth blocks' operands are in flight; the empty asm after each
+    // block keeps the compiler from requesting more than the registers hold,
+    // and from putting the block's sums off.
+    constexpr int kBlockRegs = 4 * (PW * TERMS + (SCALED ? 2 : 1) * RW);
+    constexpr int kDepth = kBlockRegs >= 48 ? 2 : 96 / kBlockRegs < kChain ? 96 / kBlockRegs : kChain;
+    bf16x8 wa[kDepth][RW], xt[kDepth][PW][TERMS];
+    float4 sc[kDepth][RW];
+    auto load = [&](int kb) {
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            wa[kb % kDepth][r] = wsrc[r][lane];
+            wsrc[r] += 64;
+            if constexpr (SCALED) {
+                sc[kb % kDepth][r] = ssrc[r][lane >> 4];
+                ssrc[r] += 4;
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < PW; p++)
+#pragma unroll
+            for (int t = 0; t < TERMS; t++) xt[kb % kDepth][p][t] = xsrc[p][t * 64 + lane];
+#pragma unroll
+        for (int p = 0; p < PW; p++) xsrc[p] += 192;
+    };
+#pragma unroll
+    for (int kb = 0; kb < kDepth; kb++) load(kb);
+#pragma unroll
+    for (int kb = 0; kb < kChain; kb++) {
+        const int at = kb % kDepth;
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            f32x4 c[PW];
+#pragma unroll
+            for (int t = 0; t < TERMS; t++)
+#pragma unroll
+                for (int p = 0; p < PW; p++)
+                    c[p] = mfma16<F16>(wa[at][r], xt[at][p][t],
+                                       t > 0 ? c[p]
+                                       : SCALED ? f32x4{0.0f, 0.0f, 0.0f, 0.0f}
+                                                : acc[r][p]);
+#pragma unroll
+            for (int p = 0; p < PW; p++) {
+                if constexpr (SCALED) {
+                    acc[r][p][0] = fmaf(sc[at][r].x, c[p][0], acc[r][p][0]);
+                    acc[r][p][1] = fmaf(sc[at][r].y, c[p][1], acc[r][p][1]);
+                    acc[r][p][2] = fmaf(sc[at][r].z, c[p][2], acc[r][p][2]);
+                    acc[r][p][3] = fmaf(sc[at][r].w, c[p][3], acc[r][p][3]);
+                } else {
+                    acc[r][p] = c[p];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+#pragma unroll
+            for (int p = 0; p < PW; p++) __asm__ volatile("" : "+v"(acc[r][p])::"memory");
+        if (kb + kDepth < kChain) load(kb + kDepth);
+    }
+    // Chain c's wave finishes tiles f with f % CHAINS == c.
+    constexpr int kMine = (kTiles + CHAINS - 1) / CHAINS;
+    EpiOperands ep[kMine];
+#pragma unroll
+    for (int i = 0; i < kMine; i++) {
+        const int f = i * CHAINS + chain, s = (pt0 + f % PW) * 16 + (lane & 15);
+        if (f >= kTiles) break;  // uniform
+        const int row0 = (rt0 + f / PW) * 16 + (lane >> 4) * 4;
+        load_epilogue_static<EPI>(ep[i], a, s, row0, s < a.streams);
+        load_epilogue_dynamic<EPI>(ep[i], a, s >> 4, s, row0, s < a.streams);
+    }
+#pragma unroll
+    for (int r = 0; r < RW; r++)
+#pragma unroll
+        for (int p = 0; p < PW; p++) part[(wave * kTiles + r * PW + p) * 64 + lane] = acc[r][p];
+    __syncthreads();
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kMine; i++) {
+        const int f = i * CHAINS + chain, s = (pt0 + f % PW) * 16 + (lane & 15);
+        if (f >= kTiles) break;  // uniform
+        const int row0 = (rt0 + f / PW) * 16 + (lane >> 4) * 4;
+        f32x4 tot = part[(wr * kTiles + f) * 64 + lane];
+#pragma unroll
+        for (int c = 1; c < CHAINS; c++) {
+            const f32x4 o = part[((c * kWr + wr) * kTiles + f) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; e++) tot[e] = __fadd_rn(tot[e], o[e]);
+        }
+        bad |= epilogue<EPI, FORMAT>(a, ep[i], tot, s, row0, s < a.streams);
+    }
     flag_nonfinite(a.status, bad);
 }
 
@@ -1054,6 +1197,177 @@ __global__ __launch_bounds__(kPairThreads) void k_prefill_attention_mfma(
 }
 
 // ---------------------------------------------------------------------------
+// Attention of short runs: one work-group per (run of up to 16 positions,
+// head). k_prefill_attention_mfma passes its keys through LDS 64 at a time,
+// two barriers and an exposed load per chunk: about 3 us each, which is what
+// bounds it when a call has few runs (25 us a layer for three prompts over
+// contexts of up to 500). Here the four waves deal the context's 16-key
+// blocks among themselves, each with an online softmax of its own, and load
+// K and V straight into the operands of the fp32 matrix cores: lane (g, n) of
+// S^T = K Q^T holds keys 4g + r of query n, which is the operand of
+// O^T += V^T P^T when step r takes keys 4g + r. The waves meet once, to merge
+// in wave order (14 us for the same three prompts; eight waves: 15). The head
+// is the grid's fast index, so that one XCD's L2 serves a (stream, head)'s
+// keys to all of its runs.
+constexpr int kShortRun = 16, kShortWaves = 4;
+
+__global__ __launch_bounds__(64 * kShortWaves) void k_prefill_attention_short(
+    const float *__restrict__ q, const float *__restrict__ kv, size_t layer_stride,
+    unsigned blocks, int layer, const int32_t *__restrict__ tables, int table_stride,
+    const int32_t *__restrict__ positions, int streams, const int32_t *__restrict__ pairs,
+    uint16_t *__restrict__ out_split, int *status) {
+    __shared__ float red[2][kShortWaves][16];
+    __shared__ float4 part[kShortWaves][4][64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4, head = blockIdx.x;
+    const int s0 = pairs[4 * blockIdx.y + 2 * blockIdx.z];
+    const int count = pairs[4 * blockIdx.y + 2 * blockIdx.z + 1];
+    if (count == 0 && blockIdx.z) return;  // uniform: the pair has one run
+    if (count < 1 || count > kShortRun || s0 < 0 || s0 > streams - count) {
+        if (threadIdx.x == 0) atomicOr(status, 2);
+        return;
+    }
+    const int32_t *table = tables + (size_t)s0 * table_stride;
+    const float *layer_kv = kv + (size_t)layer * layer_stride + (size_t)head * 2048;
+    // Block ids, 64 of the wave's blocks at a time, one per lane; the first
+    // ones are asked for before the context's length is known, like the K and V
+    // of the first blocks (every index stays inside the table and the pool).
+    int ids;
+    bool bad_block = false;
+    auto load_ids = [&](int i0) {
+        const int b = wave + kShortWaves * (i0 + lane);
+        return b < table_stride ? table[b] : 0;
+    };
+    ids = load_ids(0);
+    const int p0 = positions[s0], last = p0 + count - 1;
+    float4 qv[4];
+    const bool live = n < count;
+    {
+        const float *src = q + (size_t)(s0 + (live ? n : 0)) * kWidth + head * kHeadDim + 16 * g;
+#pragma unroll
+        for (int d = 0; d < 4; d++) qv[d] = *(const float4 *)(src + 4 * d);
+    }
+    // Key 4g + r's V row feeds step r; key n's K row the score product. kAhead
+    // blocks are in flight.
+    constexpr int kAhead = 2;
+    static_assert(64 % kAhead == 0, "the ids are reloaded between steps");
+    float4 kb[kAhead][4], vb[kAhead][4];
+    auto request = [&](int u, int i) {
+        const int id = __builtin_amdgcn_readlane(ids, i & 63);
+        const float *blk = layer_kv + (size_t)((unsigned)id < blocks ? id : 0) * kHeads * 2048;
+#pragma unroll
+        for (int d = 0; d < 4; d++) kb[u][d] = *(const float4 *)(blk + n * 64 + 16 * g + 4 * d);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            vb[u][r] = *(const float4 *)(blk + 1024 + (4 * g + r) * 64 + 4 * n);
+    };
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) request(u, u);
+    if (last / kBlockPos >= table_stride && threadIdx.x == 0) atomicOr(status, 2);
+    const int nblocks = min(last / kBlockPos + 1, table_stride);
+    const int mine = (nblocks - wave + kShortWaves - 1) / kShortWaves;  // blocks wave + 4 i
+    const int qpos = p0 + n;
+    bad_block = lane < mine && (unsigned)ids >= blocks;
+    float m = -INFINITY, l = 0.0f;
+    f32x4 o[4];  // o[d][r]: dimension 16 g + 4 r + d of query n
+#pragma unroll
+    for (int d = 0; d < 4; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto block = [&](int i, const float4 (&kc)[4], float4 (&vc)[4]) {
+        const int key0 = (wave + kShortWaves * i) * kBlockPos;
+        f32x4 sp[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) sp[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                sp[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float *)&kc[d])[u],
+                                                             ((const float *)&qv[d])[u], sp[u],
+                                                             0, 0, 0);
+        float s[4], bm = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            s[r] = key0 + 4 * g + r <= qpos
+                       ? __fadd_rn(__fadd_rn(sp[0][r], sp[1][r]), __fadd_rn(sp[2][r], sp[3][r]))
+                       : -INFINITY;
+            bm = fmaxf(bm, s[r]);
+            // Slots past the run's last position may never have been written.
+            if (key0 + 4 * g + r > last) vc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        const float mn = fmaxf(m, xor16_32_max(bm));
+        const float keep = mn == -INFINITY ? 1.0f : __expf(m - mn);
+        m = mn;
+        float ps = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            s[r] = s[r] == -INFINITY ? 0.0f : __expf(s[r] - mn);
+            ps += s[r];
+        }
+        l = fmaf(l, keep, xor16_32_sum(ps));
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+            o[d] = f32x4{o[d][0] * keep, o[d][1] * keep, o[d][2] * keep, o[d][3] * keep};
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float *)&vc[r])[d], s[r],
+                                                            o[d], 0, 0, 0);
+    };
+    for (int i0 = 0; i0 < mine; i0 += kAhead) {
+        if (((i0 + kAhead) & 63) == 0 && i0 + kAhead < mine) {
+            // The next requests are past the 64 ids held.
+            ids = load_ids(i0 + kAhead);
+            bad_block |= i0 + kAhead + lane < mine && (unsigned)ids >= blocks;
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            if (i0 + u >= mine) break;
+            block(i0 + u, kb[u], vb[u]);
+            if (i0 + u + kAhead < mine) request(u, i0 + u + kAhead);
+        }
+    }
+    if (__any(bad_block) && lane == 0) atomicOr(status, 2);
+    if (lane < 16) {
+        red[0][wave][lane] = m;
+        red[1][wave][lane] = l;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        part[wave][r][lane] = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
+    __syncthreads();
+    // Waves 0 .. 3: wave w finishes dimensions 16 g + 4 w .. + 3.
+    if (wave >= 4) return;
+    float top = red[0][0][n];
+#pragma unroll
+    for (int w = 1; w < kShortWaves; w++) top = fmaxf(top, red[0][w][n]);
+    float total = 0.0f, v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kShortWaves; w++) {
+        const float mw = red[0][w][n];
+        const float f = mw == -INFINITY ? 0.0f : __expf(mw - top);
+        const float4 a = part[w][wave][lane];
+        total = fmaf(red[1][w][n], f, total);
+        v[0] = fmaf(a.x, f, v[0]);
+        v[1] = fmaf(a.y, f, v[1]);
+        v[2] = fmaf(a.z, f, v[2]);
+        v[3] = fmaf(a.w, f, v[3]);
+    }
+    if (!live) return;
+    const bool ok = total > 0.0f && isfinite(total);
+    const float inv = 1.0f / total;
+    bool bad = !ok;
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        v[d] = ok ? v[d] * inv : 0.0f;
+        bad |= !isfinite(v[d]);
+    }
+    store_split4<true>(out_split, s0 + n, head * kHeadDim + 16 * g + 4 * wave, kWidth / 32, v,
+                       false);
+    if (bad) atomicOr(status, 1);
+}
+
+// ---------------------------------------------------------------------------
 template <int EPI, bool SCALED, int WR, int WP, int RW, int PW, int NB, int KS, int FORMAT>
 int launch_format(const GemmArgs &a, hipStream_t stream) {
     constexpr int RT = WR * RW, PT = WP * PW;
@@ -1070,6 +1384,48 @@ int launch_gemm(const GemmArgs &a, hipStream_t stream) {
     if (a.split_terms == 2)
         return launch_format<EPI, SCALED, WR, WP, RW, PW, NB, KS, 2>(a, stream);
     return launch_format<EPI, SCALED, WR, WP, RW, PW, NB, KS, 3>(a, stream);
+}
+
+template <int EPI, bool SCALED, int CHAINS, int RW, int PW>
+int launch_split(const GemmArgs &a, hipStream_t stream) {
+    const int row_groups = (a.n_rows / 16) / (RW * kTaskWaves / CHAINS);
+    const int pos_groups = ((a.streams + 15) / 16 + PW - 1) / PW;
+    hipLaunchKernelGGL((k_prefill_split<EPI, SCALED, CHAINS, RW, PW, kF16Pair>),
+                       dim3(row_groups * pos_groups), dim3(kTaskThreads), 0, stream, a,
+                       row_groups, pos_groups);
+    return launch_ok("pgpu_prefill_gemm");
+}
+
+// Up to how many 16-position tiles k_prefill_split is the faster kernel (us,
+// fp16 pairs, split / k_prefill_gemm, one box):
+//   rows           612          1024         2048         3072
+//   QKV         8.5 / 14.8  13.4 / 15.4  17.7 / 16.5  27.3 / 20.4
+//   out         5.8 / 10.0   6.0 / 10.1   7.5 / 10.4  12.5 / 11.0
+//   MLP in     12.7 / 22.9  11.8 / 22.9  19.2 / 24.2  27.6 / 25.4
+//   MLP out    10.0 / 25.4   9.8 / 25.6  16.8 / 25.8  24.0 / 26.7
+// (4096 rows: MLP out 31.2 / 29.9.) Within that: the smallest tile whose
+// work-groups still run at once, one per CU, since a work-group's time is
+// mostly the latency of its loads (24 rows, QKV: 4.8 with 1 x 1 tiles a wave,
+// 6.7 with 2 x 1, 7.5 with 2 x 2; 400 rows: 9.1, 8.8, 8.3).
+template <int EPI>
+constexpr int split_tiles(bool k2048) {
+    return EPI == EPI_QKV ? 80 : EPI == EPI_GELU_SPLIT ? 144 : k2048 ? 200 : 128;
+}
+
+template <int EPI, bool SCALED>
+int dispatch_split(const GemmArgs &a, hipStream_t stream) {
+    const int tiles = (a.streams + 15) / 16, rows = a.n_rows / 16;
+    constexpr int kFill = 256;
+    if (EPI == EPI_RESIDUAL && a.k_cols == kFfn) {
+        if (rows / 2 * tiles <= kFill)
+            return launch_split<EPI_RESIDUAL, SCALED, 8, 2, 1>(a, stream);
+        if (rows / 2 * ((tiles + 1) / 2) <= kFill)
+            return launch_split<EPI_RESIDUAL, SCALED, 8, 2, 2>(a, stream);
+        return launch_split<EPI_RESIDUAL, SCALED, 8, 4, 2>(a, stream);
+    }
+    if (rows / 4 * tiles <= kFill) return launch_split<EPI, SCALED, 2, 1, 1>(a, stream);
+    if (rows / 8 * tiles <= kFill) return launch_split<EPI, SCALED, 2, 2, 1>(a, stream);
+    return launch_split<EPI, SCALED, 2, 2, 2>(a, stream);
 }
 
 // Tile shapes (rows x positions per work-group), chosen by measurement on
@@ -1093,26 +1449,13 @@ int launch_gemm(const GemmArgs &a, hipStream_t stream) {
 //  - QKV: 192 x 64, 3 x 1 ring (1.651 against 1.717 for 192 x 128);
 //  - MLP in: 256 x 128 with a 2 x 2 ring (1.541 against 1.552 for 3 x 1,
 //    with the two above).
-// A short prompt (at most kShortPrefillTiles 16-position tiles) takes
-// 64 x 32 tiles, one MFMA tile per wave, so that its projections still
-// spread over the CUs (a 256-position prompt: 64-256 work-groups instead
-// of 16-32; a work-group's time hardly depends on its tile's size here),
-// and stages of 4 blocks (8 at K = 2048, two stages in the ring): a stage
-// costs a barrier and a copy wait whatever its size. Measured on the B=1
-// workload's 256-position prefill, 12 layers: 1.18 ms with the large tiles,
-// 0.81 with 64 x 32 tiles and 1-block stages, 0.73 with 4-block stages at
-// K = 2048, 0.70 as chosen.
-constexpr int kShortPrefillTiles = 32;
-
+// These are for many positions; fewer run on k_prefill_split.
 template <int EPI, bool SCALED>
 int dispatch_gemm(const GemmArgs &a, hipStream_t stream) {
     if (a.split_terms == kF16Pair) {
-        if ((a.streams + 15) / 16 <= kShortPrefillTiles) {
-            if constexpr (EPI == EPI_RESIDUAL)
-                if (a.k_cols == kFfn)
-                    return launch_format<EPI, SCALED, 4, 2, 1, 1, 2, 8, kF16Pair>(a, stream);
-            return launch_format<EPI, SCALED, 4, 2, 1, 1, 3, 4, kF16Pair>(a, stream);
-        }
+        if ((a.streams + 15) / 16 <= split_tiles<EPI>(a.k_cols == kFfn) &&
+            (a.k_cols == kWidth || EPI == EPI_RESIDUAL))
+            return dispatch_split<EPI, SCALED>(a, stream);
         if constexpr (EPI == EPI_GELU_SPLIT)
             if (a.n_rows % (8 * 256) == 0)
                 return launch_format<EPI, SCALED, 4, 2, 4, 4, 2, 2, kF16Pair>(a, stream);
@@ -1269,6 +1612,22 @@ extern "C" int pgpu_prefill_attention_mfma(void *stream, const float *q, const p
                            q, kv->base, kv->layer_stride, (unsigned)kv->blocks, layer, tables,
                            table_stride, positions, streams, pairs, out_split, terms, status);
     return launch_ok("pgpu_prefill_attention_mfma");
+}
+
+extern "C" int pgpu_prefill_attention_short(void *stream, const float *q, const pgpu_paged_kv *kv,
+                                            int layer, const int32_t *tables, int table_stride,
+                                            const int32_t *positions, int streams,
+                                            const int32_t *pairs, int pair_count,
+                                            uint16_t *out_split, int *status) {
+    if (!q || !kv || !tables || !positions || !pairs || !out_split || !status ||
+        streams <= 0 || layer < 0 || layer >= kv->layers || table_stride <= 0 ||
+        pair_count <= 0 || pair_count > 65535)
+        return bad_arguments("pgpu_prefill_attention_short");
+    hipLaunchKernelGGL(k_prefill_attention_short, dim3(kHeads, pair_count, 2),
+                       dim3(64 * kShortWaves), 0, (hipStream_t)stream, q, kv->base,
+                       kv->layer_stride, (unsigned)kv->blocks, layer, tables, table_stride,
+                       positions, streams, pairs, out_split, status);
+    return launch_ok("pgpu_prefill_attention_short");
 }
 
 extern "C" int pgpu_wide_from_matrix(void *stream, const pgpu_matrix *w, uint16_t *values,

@@ -8,6 +8,7 @@
  *   LN2 + MLP in projection + GELU            pgpu_gemm_gelu_split
  *   MLP out projection + residual             pgpu_gemm_residual
  * then advances every stream's position on the device. */
+#include "../csrc/pgpu_prefill.h"
 #include "ph_internal.h"
 
 #include <math.h>
@@ -55,6 +56,7 @@ struct PhononFlowBatch {
         const int32_t *pairs;       /* (dev) [pairs_count][4]: runs paired per stream (mfma) */
         int32_t *pairs_host;
         size_t pairs_count, pairs_cap;
+        int short_runs;             /* the pairs' runs are pgpu_prefill_attention_short's */
         uint16_t *split;            /* (dev) split fragments [max_streams/16][16][1536] */
         unsigned char *stage;       /* pinned host staging of a prefill call's uploads */
         unsigned char *stage_dev;   /* (dev) the same layout: one copy moves the whole area */
@@ -631,6 +633,11 @@ static int enqueue_prefill(PhononFlowBatch *b, void *stream, size_t first, size_
                                                 (int)b->table_len, b->positions, n,
                                                 b->pre.runs, (int)b->pre.runs_count, xs,
                                                 terms, b->status)
+                  : b->pre.short_runs && terms == PGPU_SPLIT_F16_PAIR
+                  ? pgpu_prefill_attention_short(stream, b->q, &b->pool->kv, layer, b->tables,
+                                                (int)b->table_len, b->positions, n,
+                                                b->pre.pairs, (int)b->pre.pairs_count, xs,
+                                                b->status)
                   : pgpu_prefill_attention_mfma(stream, b->q, &b->pool->kv, layer, b->tables,
                                                 (int)b->table_len, b->positions, n,
                                                 b->pre.pairs, (int)b->pre.pairs_count, xs,
@@ -1149,20 +1156,42 @@ static int pair_order(const void *x, const void *y) {
     return a->keys < b->keys ? 1 : (a->keys > b->keys ? -1 : (a->s0 > b->s0) - (a->s0 < b->s0));
 }
 
-/* Runs of a short prompt (at most 512 positions in the call): 16 positions,
- * so that its attention spreads over more work-groups (the B=1 workload's
- * 256-position prefill: 0.692 ms with runs of 64, 0.679 with 32, 0.674
- * with 16; a run's work-group still streams its keys once). */
-enum { PH_PREFILL_SHORT_RUN = 16 };
+/* Pairs of a list with runs of `run` positions. */
+static size_t pair_count(size_t streams, const size_t *counts, size_t run) {
+    size_t n = 0;
+    for (size_t i = 0; i < streams; i++)
+        n += ((counts[i] + run - 1) / run + 1) / 2;
+    return n;
+}
+
+/* Runs of 16 positions, for pgpu_prefill_attention_short, when runs of 64
+ * would give fewer than PH_PREFILL_MIN_PAIRS pairs, i.e. work-groups for less
+ * than half the CUs (8 per pair). A 12-layer call, us, short against long
+ * runs: 3 prompts / 611 positions 797 / 947, 4 / 1024 814 / 898, 6 / 1613 over
+ * contexts of up to 900 1364 / 1455 (14 pairs); 8 / 2048 1305 / 1293 (16);
+ * 16 / 4096 2250 / 2083; 10 / 3523 over contexts of up to 1100 2768 / 2592.
+ * Without fp16 weights (pgpu_prefill_attention_mfma either way): at most 512
+ * positions, so that a short prompt spreads over more work-groups. */
+enum { PH_PREFILL_SHORT_RUN = 16, PH_PREFILL_MIN_PAIRS = 16, PH_PREFILL_SHORT_TOTAL = 512 };
+
+/* Every layer of the model runs its fast prefill on fp16 pairs. */
+static int prefill_f16(const PhononFlowModel *m) {
+    for (size_t i = 0; i < m->layers * 4; i++)
+        if (!m->wide[i].values_f16)
+            return 0;
+    return 1;
+}
 
 static int prefill_pairs(PhononFlowBatch *b, size_t streams, const size_t *first,
                          const size_t *counts) {
-    size_t n = 0, total = 0;
+    size_t total = 0;
     for (size_t i = 0; i < streams; i++)
         total += counts[i];
-    const size_t run = total <= 512 ? PH_PREFILL_SHORT_RUN : PH_PREFILL_RUN;
-    for (size_t i = 0; i < streams; i++)
-        n += ((counts[i] + run - 1) / run + 1) / 2;
+    b->pre.short_runs = prefill_f16(b->model) &&
+                        pair_count(streams, counts, PH_PREFILL_RUN) < PH_PREFILL_MIN_PAIRS;
+    const size_t run = b->pre.short_runs || total <= PH_PREFILL_SHORT_TOTAL ? PH_PREFILL_SHORT_RUN
+                                                                            : PH_PREFILL_RUN;
+    size_t n = pair_count(streams, counts, run);
     PrefillPair *list = malloc(n * sizeof(PrefillPair));
     if (!list)
         return 0;

@@ -914,6 +914,60 @@ def test_fast_prefill_around_the_short_prompt_path(lib, syn, pkg, counts, first)
     assert worst <= 1e-4
 
 
+@pytest.mark.parametrize("counts,first", [
+    ([1], [0]), ([17, 3], [0, 5]), ([129], [0]), ([250, 91], [0, 33]), ([40, 16], [4190, 63]),
+    ([70] * 15, [1] * 15), ([70] * 16, [1] * 16), ([1281], [0]), ([2049], [0]), ([2320], [0]),
+    ([3216], [0])])
+def test_fast_prefill_tiles_and_runs(lib, syn, pkg, counts, first):
+    """Calls on both sides of the fast prefill's choices: one position and
+    ragged tails, each projection tile (wave tiles of 1 x 1, 2 x 1 and 2 x 2,
+    and where the many-position kernels take over), short attention runs over
+    contexts of more than 64 blocks a wave, 15 and 16 pairs of long runs. The
+    exact prefill of the same call is the reference: every row within 1e-4
+    normwise."""
+    layers, nstreams, total = 2, len(counts), sum(counts)
+    model, views = scaled_model(syn, 193, layers), pkg.Views()
+    w = views.layers(model)
+    need = [-(-(a + b) // 16) for a, b in zip(counts, first)]
+    table_len, blocks = max(need), sum(need)
+    rng = np.random.default_rng(194)
+    past = max(first)
+    ctx = rng.standard_normal((2, layers, max(past, 1), 512)).astype(np.float32)
+    x = rng.standard_normal((total, 512)).astype(np.float32)
+    szp = ctypes.POINTER(ctypes.c_size_t)
+    f, c = np.array(first, np.uintp), np.array(counts, np.uintp)
+    outs = []
+    for exact in (1, 0):
+        bt = Batch(lib, w, layers, total, 16 * table_len, blocks)
+        ids = np.zeros(blocks, np.int32)
+        assert lib.phonon_kv_pool_alloc(bt.pool, blocks, i32p(ids))
+        ids = np.random.default_rng(195).permutation(ids).astype(np.int32)
+        tables, at = np.zeros((nstreams, table_len), np.int32), 0
+        for i, n in enumerate(need):
+            tables[i, :n] = ids[at:at + n]
+            at += n
+            if first[i]:
+                assert lib.phonon_kv_pool_write(bt.pool, i32p(tables[i]), table_len, 0, first[i],
+                                                fp(ctx[0]), fp(ctx[1]), past)
+        assert lib.phonon_flow_batch_set_prefill_exact(bt.batch, exact)
+        din = pkg.DeviceBuffer(lib, total * 512 * 4)
+        dout = pkg.DeviceBuffer(lib, total * 512 * 4)
+        din.upload(x)
+        assert lib.phonon_flow_batch_prefill_device(bt.batch, nstreams, f.ctypes.data_as(szp),
+                                                    c.ctypes.data_as(szp), i32p(tables),
+                                                    table_len, din.ptr, 10000.0, dout.ptr), \
+            pkg.last_error(lib)
+        assert lib.phonon_flow_batch_sync(bt.batch)
+        outs.append(dout.download((total, 512)))
+        din.free()
+        dout.free()
+        bt.close()
+    assert np.all(np.isfinite(outs[1]))
+    worst = max(helpers.normwise(b, a) for a, b in zip(outs[0], outs[1]))
+    print(f"fast prefill of {counts} at {first} vs exact: max normwise {worst:.3g}", flush=True)
+    assert worst <= 1e-4
+
+
 def test_prefill_calls_enqueued_back_to_back(lib, syn, pkg):
     """Prefill calls enqueued one after another with no wait between them
     give the bits of the same calls with a synchronize after each: three
