@@ -3,6 +3,7 @@
 // of phonon_transformer.h / phonon_q8.h and by the batched step when it runs
 // phase by phase; the one-launch step (pgpu_flow.hip) runs the same tasks.
 #include "pgpu_gemm.hpp"
+#include "pgpu_gemm_rows.h"
 #include "phonon_gpu.h"
 
 namespace pgpu {
@@ -17,6 +18,71 @@ template <int SRC, int EPI, bool Q8>
 __global__ __launch_bounds__(kTaskThreads) void k_gemm_wide(GemmArgs a) {
     __shared__ uint4 bsh4[kTaskLds / 8];
     gemm_wide_task<SRC, EPI, Q8>(a, blockIdx.x, blockIdx.y, (uint16_t *)bsh4, NoWait{});
+}
+
+// gemm_split_task on fp32 rows (a.ln_x, [streams][k_cols]): a lane splits its
+// 8 columns of each block itself, all 8 blocks of its wave's range (K = 2048)
+// requested at once. Every row tile's work-group splits the rows again, which
+// is less than the launch that would do it for them: a 512 x 2048 product of
+// one row is bound by its launches and load latencies (7.5 us with the rows
+// split by a launch of their own, 5.2 with this).
+template <bool Q8>
+__global__ __launch_bounds__(kTaskThreads) void k_gemm_rows(GemmArgs a) {
+    constexpr int CH = 8;
+    __shared__ f32x4 partial[kTaskWaves * 64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, tile = blockIdx.x, st = blockIdx.y;
+    const int kbn = a.k_cols >> 5, per = (kbn + kTaskWaves - 1) / kTaskWaves;
+    const int kb_begin = wave * per, kb_end = min(kbn, kb_begin + per);
+    const int s = st * 16 + (lane & 15), row0 = tile * 16 + (lane >> 4) * 4;
+    const bool live = s < a.streams;
+    const float *row = a.ln_x + (size_t)(live ? s : 0) * a.k_cols + 8 * (lane >> 4);
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    bool bad = false;
+    for (int kb0 = kb_begin; kb0 < kb_end; kb0 += CH) {
+        WChunk<Q8, CH> w;
+        load_weights(w, a, tile, kbn, lane, kb0, kb_end);
+        float4 x[CH][2];
+#pragma unroll
+        for (int u = 0; u < CH; u++) {
+            const float4 *src = (const float4 *)(row + min(kb0 + u, kb_end - 1) * 32);
+            x[u][0] = src[0];
+            x[u][1] = src[1];
+        }
+#pragma unroll
+        for (int u = 0; u < CH; u++) {
+            const float v[8] = {x[u][0].x, x[u][0].y, x[u][0].z, x[u][0].w,
+                                x[u][1].x, x[u][1].y, x[u][1].z, x[u][1].w};
+            uint16_t h[8], m[8], l[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                bad |= live && !isfinite(v[k]);
+                split3(live ? v[k] : 0.0f, h[k], m[k], l[k]);
+            }
+            auto pack = [](const uint16_t *t) {
+                return __builtin_bit_cast(bf16x8, make_uint4(t[0] | (uint32_t)t[1] << 16,
+                                                             t[2] | (uint32_t)t[3] << 16,
+                                                             t[4] | (uint32_t)t[5] << 16,
+                                                             t[6] | (uint32_t)t[7] << 16));
+            };
+            mfma_block(acc, w, u, pack(h), pack(m), pack(l), kb0 + u < kb_end);
+        }
+    }
+    partial[wave * 64 + lane] = acc;
+    __syncthreads();
+    if (wave == 0) {
+        f32x4 v = acc;
+#pragma unroll
+        for (int w = 1; w < kTaskWaves; w++) {
+            const f32x4 p = partial[w * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = __fadd_rn(v[r], p[r]);
+        }
+        EpiOperands e;
+        load_epilogue_static<EPI_STORE>(e, a, s, row0, live);
+        bad |= epilogue<EPI_STORE>(a, e, v, s, row0, live);
+    }
+    flag_nonfinite(a.status, bad);
 }
 
 template <int SRC, int EPI, bool Q8>
@@ -95,6 +161,23 @@ extern "C" int pgpu_gemm_store(void *stream, const pgpu_matrix *w, const pgpu_ge
     a.ld_out = ld_out;
     a.bias = bias;
     return dispatch<EPI_STORE>(a, w->q8, (hipStream_t)stream);
+}
+
+extern "C" int pgpu_gemm_store_rows(void *stream, const pgpu_matrix *w, const float *rows,
+                                    int streams, float *out, int ld_out, int *status) {
+    GemmArgs a;
+    const pgpu_gemm_input in = {.rows = rows};
+    if (!w || !rows || !out || !status || streams <= 0 || !w->rows || w->rows % 16 ||
+        !w->columns || w->columns % 32 || !base_args(a, w, &in, streams, status))
+        return bad_arguments("pgpu_gemm_store_rows");
+    a.out = out;
+    a.ld_out = ld_out;
+    const dim3 grid(a.n_rows / 16, (streams + 15) / 16);
+    if (w->q8)
+        hipLaunchKernelGGL(k_gemm_rows<true>, grid, dim3(kTaskThreads), 0, (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL(k_gemm_rows<false>, grid, dim3(kTaskThreads), 0, (hipStream_t)stream, a);
+    return launch_ok("pgpu_gemm_store_rows");
 }
 
 extern "C" int pgpu_gemm_residual(void *stream, const pgpu_matrix *w, const pgpu_gemm_input *in,

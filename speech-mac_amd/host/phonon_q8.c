@@ -10,6 +10,7 @@
  * pgpu_gemm.hip), and the drop-in matvec falls back to that path when the
  * column count is not 32 x a divisor of 64. */
 #include "phonon_q8_device.h"
+#include "../csrc/pgpu_gemm_rows.h"
 #include "ph_internal.h"
 
 #include <stdlib.h>
@@ -116,6 +117,10 @@ int phonon_q8_device_matvec(PhononQ8Device *m, size_t copy, const float *x, floa
         const pgpu_gemm_input rows = {.rows = x};
         return pgpu_gemm_store(stream, w, &rows, (int)batch, NULL, y, (int)w->rows, m->status);
     }
+    /* One launch for other widths too; an output that overlaps the input needs
+     * the rows read before any result is written. */
+    if (!ph_overlap(x, batch * w->columns * sizeof(float), y, batch * w->rows * sizeof(float)))
+        return pgpu_gemm_store_rows(stream, w, x, (int)batch, y, (int)w->rows, m->status);
     const pgpu_gemm_input in = {.split = m->xs};
     return pgpu_split_rows(stream, x, (int)batch, (int)w->columns, m->xs, m->status) &&
            pgpu_gemm_store(stream, w, &in, (int)batch, NULL, y, (int)w->rows, m->status);

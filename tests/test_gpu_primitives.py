@@ -153,6 +153,35 @@ def test_q8_device_matvec_512_columns_rows_path(lib, oracle, syn, pkg, batch):
     lib.phonon_q8_device_destroy(handle)
 
 
+@pytest.mark.parametrize("rows,cols,batch", [
+    (16, 32, 1), (48, 64, 3), (512, 2048, 16), (512, 2048, 17), (32, 2080, 2), (64, 4128, 33)])
+def test_q8_device_matvec_rows_split_in_the_product(lib, syn, pkg, rows, cols, batch):
+    """Widths other than 512 split their rows inside the product: block counts
+    below, at and past the eight a wave requests at once, odd ones, and whole and
+    partial 16-row tiles. The bits of the rows split by a launch of their own,
+    which an output laid over the input still takes; a non-finite input is
+    reported."""
+    rng = np.random.default_rng(rows + cols)
+    w = syn.q8_matrix(rng, rows, cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    handle = ctypes.c_void_p()
+    assert lib.phonon_q8_device_create(w.ctypes.data, rows, cols, 1, ctypes.byref(handle))
+    dx = pkg.DeviceBuffer(lib, max(cols, rows) * batch * 4)
+    dy = pkg.DeviceBuffer(lib, batch * rows * 4)
+    dx.upload(x)
+    assert lib.phonon_q8_device_matvec(handle, 0, dx.ptr, dy.ptr, batch, None)
+    assert lib.phonon_q8_device_status(handle, None)
+    y = dy.download((batch, rows))
+    assert lib.phonon_q8_device_matvec(handle, 0, dx.ptr, dx.ptr, batch, None)
+    assert lib.phonon_q8_device_status(handle, None)
+    assert np.array_equal(bits(dx.download((batch, rows))), bits(y))
+    x[batch - 1, cols - 1] = np.inf
+    dx.upload(x)
+    assert lib.phonon_q8_device_matvec(handle, 0, dx.ptr, dy.ptr, batch, None)
+    assert not lib.phonon_q8_device_status(handle, None)
+    lib.phonon_q8_device_destroy(handle)
+
+
 @pytest.mark.parametrize("rows,cols", [(2048, 512), (512, 2048), (48, 64)])
 @pytest.mark.parametrize("batch", [1, 2, 5, 8])
 def test_q8_device_matvec_valu_bits(lib, oracle, syn, pkg, rows, cols, batch):
