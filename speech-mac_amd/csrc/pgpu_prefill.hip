@@ -1295,12 +1295,12 @@ __global__ __launch_bounds__(64 * kShortWaves) void k_prefill_attention_short(
             if (key0 + 4 * g + r > last) vc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         const float mn = fmaxf(m, xor16_32_max(bm));
-        const float keep = mn == -INFINITY ? 1.0f : __expf(m - mn);
+        const float keep = mn == -INFINITY ? 1.0f : expf(m - mn);
         m = mn;
         float ps = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            s[r] = s[r] == -INFINITY ? 0.0f : __expf(s[r] - mn);
+            s[r] = s[r] == -INFINITY ? 0.0f : expf(s[r] - mn);
             ps += s[r];
         }
         l = fmaf(l, keep, xor16_32_sum(ps));
@@ -1345,7 +1345,7 @@ __global__ __launch_bounds__(64 * kShortWaves) void k_prefill_attention_short(
 #pragma unroll
     for (int w = 0; w < kShortWaves; w++) {
         const float mw = red[0][w][n];
-        const float f = mw == -INFINITY ? 0.0f : __expf(mw - top);
+        const float f = mw == -INFINITY ? 0.0f : expf(mw - top);
         const float4 a = part[w][wave][lane];
         total = fmaf(red[1][w][n], f, total);
         v[0] = fmaf(a.x, f, v[0]);
