@@ -146,7 +146,7 @@ int phonon_flow_batch_set_trace(PhononFlowBatch *batch, uint64_t *trace, size_t 
 size_t phonon_flow_batch_schedule(const PhononFlowBatch *batch, uint32_t *schedule,
                                   size_t capacity);
 /* One-launch step: 256-key attention splits per ATTN task (1 or 2; 0, the
- * default: chosen by the batch size). Results are identical for every
+ * default: chosen by the batch size and its contexts). Results are identical for every
  * choice. */
 int phonon_flow_batch_set_attention_rounds(PhononFlowBatch *batch, int rounds);
 /* One-launch step: how tasks hand the layer output, the out projection,

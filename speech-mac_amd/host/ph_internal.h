@@ -26,16 +26,10 @@ enum { PH_PREFILL_RUN = PGPU_PREFILL_RUN, PH_PREFILL_MIN_GROUPS = 1024 };
  * 1450; B = 192: 1954 vs 2076; B = 224: 2277 vs 2347; B = 256: 2649 vs
  * 2642). */
 enum { PH_FLOW_MIN_TILES = 1, PH_FLOW_MAX_TILES = 14 };
-/* One-launch steps of at most PH_FLOW_ONE_ROUND_MAX_STREAMS streams, or of
- * PH_FLOW_ONE_ROUND_MIN_TILES..PH_FLOW_ONE_ROUND_MAX_TILES tiles, run one
- * split per ATTN task (the others PGPU_FLOW_ATTN_ROUNDS): us per step, one
- * vs two splits, B = 32: 674 vs 552; B = 48: 693 vs 712; B = 64: 680 vs
- * 689; B = 80: 890 vs 834. */
-enum {
-    PH_FLOW_ONE_ROUND_MAX_STREAMS = 8,
-    PH_FLOW_ONE_ROUND_MIN_TILES = 3,
-    PH_FLOW_ONE_ROUND_MAX_TILES = 4
-};
+/* One-launch steps of at most this many streams, or of at most this many
+ * attention splits over all heads, run one split per ATTN task (the others
+ * PGPU_FLOW_ATTN_ROUNDS; flow_rounds has the measurements). */
+enum { PH_FLOW_ONE_ROUND_MAX_STREAMS = 8, PH_FLOW_ONE_ROUND_MAX_SPLITS = 3600 };
 /* One-launch steps of at most this many streams hand values over as tagged
  * words (phonon_flow_batch_set_handoff). */
 enum { PH_FLOW_TAGGED_MAX_STREAMS = 4 };

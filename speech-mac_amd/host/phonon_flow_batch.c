@@ -82,7 +82,8 @@ struct PhononFlowBatch {
         size_t *cover;              /* [max_streams] splits the schedule lists per stream */
         size_t *units;              /* [max_streams] ATTN tasks per (stream, head) for them */
         int rounds;                 /* splits per ATTN task the schedule was built for */
-        int rounds_set;             /* 0: by batch size, else the caller's choice */
+        int rounds_set;             /* 0: by batch and contexts, else the caller's choice */
+        int rounds_for;             /* rounds_set when the schedule was built */
         int place_set;              /* the caller set the placement */
         size_t streams, layers;     /* what the schedule was built for (0: none) */
         int prefill, fused;
@@ -792,17 +793,40 @@ static size_t flow_ml_group(const PhononFlowBatch *b) {
  * than one launch per phase (PH_FLOW_MIN_TILES..PH_FLOW_MAX_TILES 16-stream
  * tiles; prefill and larger batches are attention-bound, where the separate
  * attention kernel streams K/V faster). */
-/* Splits per ATTN task: one for a few streams (the step is a latency
- * chain) and at 3 and 4 tiles, two otherwise (fewer, longer attention tasks
- * keep more K/V in flight per work-group slot); measured on MI355X. */
-static int flow_rounds(const PhononFlowBatch *b) {
+/* Splits per ATTN task of a step that lists `splits` of them per head: one
+ * while a step is a latency chain, two (fewer, longer attention tasks, which
+ * keep more K/V in flight per work-group slot) once it streams. us per step,
+ * one / two, contexts U{1..n}: 16 streams n = 1000 443 / 469; 24, 2048 538 /
+ * 551; 48, 2048 636 / 686; 64, 2048 (3248 splits in all) 730 / 795; 80, 2048
+ * (3920) 865 / 814; 64, 6000 (6928) 1585 / 1511. Up to two tiles whose
+ * contexts fill one task of two splits run those (12 streams, n = 300: 369 /
+ * 364), except the smallest batches. */
+static int flow_rounds(const PhononFlowBatch *b, size_t splits) {
     if (b->fl.rounds_set)
         return b->fl.rounds_set;
     const size_t tiles = (b->streams + 15) / 16;
-    return b->streams <= PH_FLOW_ONE_ROUND_MAX_STREAMS ||
-                   (tiles >= PH_FLOW_ONE_ROUND_MIN_TILES && tiles <= PH_FLOW_ONE_ROUND_MAX_TILES)
-               ? 1
-               : PGPU_FLOW_ATTN_ROUNDS;
+    if (b->streams <= PH_FLOW_ONE_ROUND_MAX_STREAMS)
+        return 1;
+    if (tiles <= 2 && splits <= 2 * b->streams)
+        return PGPU_FLOW_ATTN_ROUNDS;
+    return splits * PH_HEADS <= PH_FLOW_ONE_ROUND_MAX_SPLITS ? 1 : PGPU_FLOW_ATTN_ROUNDS;
+}
+
+/* Where a decode step lists a tile's chain: its QKV, the last of the four
+ * phases, just before the other tiles' attention tasks of the layer run out,
+ * for that is when the tile's next attention can be listed; the others before
+ * it in the proportion of the times they take. An offset that does not follow
+ * the contexts lists the chain too late for short ones (its tile starves) and
+ * too early for long ones (waiting tasks hold slots). us per step, contexts
+ * U{1..n}, against offsets that were the same for all (550 .. 1750 tasks): 24
+ * streams n = 6000 801 / 894; 40, 2048 603 / 744; 48, 2048 636 / 755; 64, 300
+ * 462 / 612; 64, 2048 730 / 735; 64, 6000 1511 / 1725; 96, 300 463 / 711; 128,
+ * 600 578 / 667. The share of the others' tasks: swept 0.7 .. 1.06; the best
+ * lies at 0.94 .. 1 up to 2800 splits and at 0.76 .. 0.88 beyond. */
+static pgpu_flow_placement flow_placement(size_t tiles, size_t splits, int rounds) {
+    const double others = (double)splits * (tiles - 1) / tiles;
+    const float last = (float)(others * (splits <= 2800 ? 0.94 : 0.82));
+    return (pgpu_flow_placement){(float)rounds, {0.314f * last, 0.571f * last, 0.829f * last, last}};
 }
 
 static int flow_usable(const PhononFlowBatch *b, int prefill) {
@@ -912,24 +936,32 @@ static int flow_mode(const PhononFlowBatch *b, int prefill) {
  * end at once. */
 static int flow_schedule(PhononFlowBatch *b, int prefill) {
     const size_t streams = b->streams, layers = b->model->layers;
-    const int rounds = flow_rounds(b);
     const int fused = flow_mode(b, prefill) == PGPU_FLOW_HANDOFF_FUSED_MLP;
     const int flags = (prefill ? PGPU_FLOW_SCHEDULE_PREFILL : 0) |
                       (fused ? PGPU_FLOW_SCHEDULE_FUSED_MLP : 0);
     int valid = b->fl.streams == streams && b->fl.layers == layers && b->fl.prefill == prefill &&
-                b->fl.rounds == rounds && b->fl.fused == fused;
+                b->fl.rounds_for == b->fl.rounds_set && b->fl.fused == fused;
     for (size_t s = 0; valid && s < streams; s++)
         valid = (b->host_positions[s] + PH_SPLIT_KEYS) / PH_SPLIT_KEYS <= b->fl.cover[s];
     if (valid)
         return 1;
     b->fl.streams = 0; /* no valid schedule until the new one is uploaded */
+    size_t splits = 0;
     for (size_t s = 0; s < streams; s++) {
         size_t need = (b->host_positions[s] + PH_FLOW_HEADROOM + PH_SPLIT_KEYS) / PH_SPLIT_KEYS;
         b->fl.cover[s] = need < b->max_splits ? need : b->max_splits;
+        splits += b->fl.cover[s];
+    }
+    const int rounds = flow_rounds(b, splits);
+    splits = 0;
+    for (size_t s = 0; s < streams; s++) {
         b->fl.units[s] = (b->fl.cover[s] + rounds - 1) / rounds;
+        splits += b->fl.units[s] * rounds;
     }
     const pgpu_flow_placement place =
-        b->fl.place_set ? b->fl.place : ph_flow_default_placement(rounds);
+        b->fl.place_set ? b->fl.place
+        : prefill       ? ph_flow_default_placement(rounds)
+                        : flow_placement((streams + 15) / 16, splits * PH_HEADS, rounds);
     const size_t tasks =
         pgpu_flow_schedule(streams, layers, b->fl.units, &place, flags, NULL, 0);
     if (tasks > b->fl.host_cap) {
@@ -957,6 +989,7 @@ static int flow_schedule(PhononFlowBatch *b, int prefill) {
     if (!pgpu_copy_h2d(b->stream, b->fl.schedule, d, tasks * sizeof(uint32_t)))
         return 0;
     b->fl.rounds = rounds;
+    b->fl.rounds_for = b->fl.rounds_set;
     b->fl.tasks = tasks;
     b->fl.streams = streams;
     b->fl.layers = layers;

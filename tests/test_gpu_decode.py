@@ -1079,6 +1079,37 @@ def test_one_launch_step_equals_phase_launches(lib, syn, pkg, streams):
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("streams,high", [(12, 200), (12, 1200), (24, 4000), (40, 200), (70, 900),
+                                          (96, 4000)])
+def test_schedule_follows_the_contexts(lib, syn, pkg, streams, high):
+    """The default step lists one or two attention splits per task and places a
+    tile's chain by the contexts: few and many splits for one tile, for several,
+    and past the line to two per task. The bits of the layers phase by phase."""
+    layers = 2
+    model, views = scaled_model(syn, 185, layers), pkg.Views()
+    w = views.layers(model)
+    lengths = np.random.default_rng(186).integers(1, high + 1, streams).astype(np.uintp)
+    table_len = -(-(high + 8) // 16)
+    x = np.random.default_rng(187).standard_normal((streams, 512)).astype(np.float32)
+    outs = []
+    for flow in (0, 1):
+        bt = Batch(lib, w, layers, streams, 16 * table_len, streams * table_len)
+        assert lib.phonon_kv_pool_fill_normal(bt.pool, 188)
+        assert lib.phonon_flow_batch_set_pipeline(bt.batch, flow)
+        ids = np.zeros(streams * table_len, np.int32)
+        assert lib.phonon_kv_pool_alloc(bt.pool, ids.size, i32p(ids))
+        tables = np.ascontiguousarray(ids.reshape(streams, table_len))
+        assert lib.phonon_flow_batch_set_streams(
+            bt.batch, streams, lengths.ctypes.data_as(ctypes.POINTER(ctypes.c_size_t)),
+            i32p(tables), table_len)
+        for _ in range(2):
+            y = np.zeros((streams, 512), np.float32)
+            assert lib.phonon_flow_batch_step(bt.batch, fp(x), 10000.0, fp(y)), pkg.last_error(lib)
+            outs.append(y.view(np.uint32))
+        bt.close()
+    assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[3])
+
+
 @pytest.mark.parametrize("streams", [1, 2, 4])
 def test_fused_mlp_step_vs_oracle(lib, oracle, oracle_mod, syn, pkg, streams):
     """The fused-MLP hand-off (mode 4: no MLP-out phase; each MLP-in task's
