@@ -670,8 +670,11 @@ void launch_product(hipStream_t st, const pgpu_plane_product &a, const pgpu_plan
 // Short passes are bound by latency, long ones by what the work-groups read
 // from L2: per reduction index a tile reads 2 bytes a column and 6 a position,
 // so tiles are wide in columns, and a larger one is taken as soon as it
-// leaves enough work-groups. conv0's seven taps of weights would not fit the
-// registers of a 64-column tile.
+// leaves enough work-groups (us, 4 x 4 / 2 x 4 tiles: 512 positions, 1536
+// columns, K = 1024 14.0 / 10.8 at 192 groups of the larger; 1024 positions,
+// 2048 columns, K = 512 16.4 / 18.9 at 512). conv0's seven taps of weights
+// would not fit the registers of a 64-column tile; 4 x 2 took 22.8 us at 1024
+// positions, 2 x 2 takes 16.9.
 template <int EPI>
 void launch_tile(hipStream_t st, const pgpu_plane_product &a, const pgpu_planes &in,
                  int positions, pgpu_pass pass, int *status) {
@@ -679,12 +682,10 @@ void launch_tile(hipStream_t st, const pgpu_plane_product &a, const pgpu_planes 
         return (long)((positions + 16 * pt - 1) / (16 * pt)) * (a.ncols / (16 * ct));
     };
     if constexpr (EPI == PGPU_PLANE_ELU) {
-        if (groups(4, 2) >= 224)
-            return launch_product<EPI, 4, 2>(st, a, in, positions, pass, status);
         if (groups(2, 2) >= 96)
             return launch_product<EPI, 2, 2>(st, a, in, positions, pass, status);
     } else {
-        if (groups(4, 4) >= 192)
+        if (groups(4, 4) >= 384)
             return launch_product<EPI, 4, 4>(st, a, in, positions, pass, status);
         if (groups(2, 4) >= 160)
             return launch_product<EPI, 2, 4>(st, a, in, positions, pass, status);
@@ -832,10 +833,8 @@ extern "C" int pgpu_pcm_residual(void *stream, const pgpu_residual_weights *w, i
         else
             launch_residual<256, 2>(st, *w, x, positions, pass, history, out, pcm, status);
     } else if (channels == 128) {
-        if (positions <= 32 * 256)
-            launch_residual<128, 2>(st, *w, x, positions, pass, history, out, pcm, status);
-        else
-            launch_residual<128, 4>(st, *w, x, positions, pass, history, out, pcm, status);
+        // (64-position groups: 21.1 us at 29,760 positions, these 18.4.)
+        launch_residual<128, 2>(st, *w, x, positions, pass, history, out, pcm, status);
     } else {
         launch_residual<64, 4>(st, *w, x, positions, pass, history, out, pcm, status);
     }
