@@ -13,6 +13,7 @@
 #include <cmath>
 
 #include "pgpu_gemm.hpp"
+#include "pgpu_head.h"
 #include "phonon_gpu.h"
 
 namespace pgpu {
@@ -106,10 +107,15 @@ __global__ __launch_bounds__(kTaskThreads) void k_head_mod(GemmArgs ada, GemmArg
 }
 
 // A block's first MLP projection with its LayerNorm and modulation fused in
-// front: split fragments of SiLU(mlp_0(LN(x) * (1 + scale) + shift)).
-__global__ __launch_bounds__(kTaskThreads) void k_head_mlp_in(GemmArgs a) {
+// front: split fragments of SiLU(mlp_0(LN(x) * (1 + scale) + shift)). It is
+// 8 work-groups per 16 streams, so the adaLN rows that the next block (or the
+// final layer) needs can be computed beside it: the second launch then holds
+// one block's, 224 work-groups at 64 streams instead of 768 in two rounds.
+__global__ __launch_bounds__(kTaskThreads) void k_head_mlp_in(GemmArgs a, GemmArgs ada) {
     __shared__ uint4 lds4[kTaskLds / 8];
-    wide_at<SRC_LN_MOD, EPI_SILU_SPLIT>(a, blockIdx.x, (uint16_t *)lds4);
+    const int b = blockIdx.x, n = wide_groups(a);
+    if (b < n) return wide_at<SRC_LN_MOD, EPI_SILU_SPLIT>(a, b, (uint16_t *)lds4);
+    wide_at<SRC_SPLIT_LDS, EPI_STORE>(ada, b - n, (uint16_t *)lds4);
 }
 
 // A residual block of the fused chain, one launch: x (the rows, SRC_LN_MOD,
@@ -291,13 +297,17 @@ extern "C" int pgpu_head_mod(void *stream, const pgpu_matrix *ada_w, const uint1
     return launch_ok(__func__);
 }
 
-extern "C" int pgpu_head_mlp_in(void *stream, const pgpu_matrix *w, const float *x, int streams,
-                                const float *norm_w, const float *norm_b, float eps,
-                                const float *mod, int ld_mod, const float *bias,
-                                uint16_t *out_split, int *status) {
+extern "C" int pgpu_head_mlp_in_beside(void *stream, const pgpu_matrix *w, const float *x,
+                                       int streams, const float *norm_w, const float *norm_b,
+                                       float eps, const float *mod, int ld_mod, const float *bias,
+                                       uint16_t *out_split, const pgpu_matrix *next_ada,
+                                       const uint16_t *silu_split, const float *next_bias,
+                                       float *next_mod, int *status) {
     if (!bf16_matrix(w, kWidth, kWidth) || !x || streams <= 0 || !mod || ld_mod < 2 * kWidth ||
-        ld_mod % 4 || !out_split || !(eps > 0.0f))
-        return bad_arguments(__func__);
+        ld_mod % 4 || !out_split || !(eps > 0.0f) ||
+        (next_ada && (!bf16_matrix(next_ada, next_ada->rows, kWidth) || next_ada->rows % 16 ||
+                      !silu_split || !next_mod || ld_mod < (int)next_ada->rows)))
+        return bad_arguments("pgpu_head_mlp_in");
     GemmArgs a = head_args(w, streams, status);
     a.ln_x = x;
     a.ln_w = norm_w;
@@ -308,9 +318,26 @@ extern "C" int pgpu_head_mlp_in(void *stream, const pgpu_matrix *w, const float 
     a.bias = bias;
     a.out_split = out_split;
     a.out_kb = kWidth / 32;
-    hipLaunchKernelGGL(k_head_mlp_in, dim3((unsigned)wide_groups(a)), dim3(kTaskThreads), 0,
-                       (hipStream_t)stream, a);
-    return launch_ok(__func__);
+    GemmArgs ada{};
+    if (next_ada) {
+        ada = head_args(next_ada, streams, status);
+        ada.xs = silu_split;
+        ada.bias = next_bias;
+        ada.out = next_mod;
+        ada.ld_out = ld_mod;
+    }
+    const int blocks = wide_groups(a) + (next_ada ? wide_groups(ada) : 0);
+    hipLaunchKernelGGL(k_head_mlp_in, dim3((unsigned)blocks), dim3(kTaskThreads), 0,
+                       (hipStream_t)stream, a, ada);
+    return launch_ok("pgpu_head_mlp_in");
+}
+
+extern "C" int pgpu_head_mlp_in(void *stream, const pgpu_matrix *w, const float *x, int streams,
+                                const float *norm_w, const float *norm_b, float eps,
+                                const float *mod, int ld_mod, const float *bias,
+                                uint16_t *out_split, int *status) {
+    return pgpu_head_mlp_in_beside(stream, w, x, streams, norm_w, norm_b, eps, mod, ld_mod, bias,
+                                   out_split, nullptr, nullptr, nullptr, nullptr, status);
 }
 
 // The previous block's partials (pgpu_head_parts) checked and set into a.

@@ -14,6 +14,7 @@
  * depend on the stream: tsum = 0.5 (time_0(0) + time_1(1)) is computed once
  * on the device when the head is created. */
 #include "phonon_sampler.h"
+#include "../csrc/pgpu_head.h"
 #include "ph_internal.h"
 
 #include <math.h>
@@ -358,6 +359,16 @@ static int enqueue_tsum(PhononFlowHeadDevice *h, float s, float t, float *tsum) 
                               h->alpha[1], tsum, h->status);
 }
 
+enum { SPREAD_STREAMS = 32 };
+
+/* `count` modulation columns from `first` on, as a projection of their own. */
+static pgpu_matrix ada_rows(const PhononFlowHeadDevice *h, size_t first, size_t count) {
+    pgpu_matrix w = h->ada;
+    w.values = (const uint16_t *)w.values + first * PH_WIDTH;
+    w.rows = count;
+    return w;
+}
+
 /* The head for n streams: conditions [n][512], raw [n][32] scaled by `scale`
  * (out_split: the latent's split fragments too, lsd only)
  * into the state (the noise of an LSD step, or the normalized state itself
@@ -370,15 +381,23 @@ static int enqueue_head(PhononFlowHeadDevice *h, size_t n, const float *conditio
                         PhononCancelPoll cancel, void *context) {
     void *st = h->stream;
     const int B = (int)n;
+    const int fused = h->fused > 0 || (h->fused < 0 && n <= FUSED_AUTO_STREAMS);
     const pgpu_gemm_input first = {.split = h->first_split};
+    /* From three tiles on, all of the modulation in one launch is more than one
+     * round of work-groups: block 0's goes first and each next part beside a
+     * block's MLP (us per frame, 33 streams 84.4 -> 81.4, 64 84.8 -> 82.4, 256
+     * 109 -> 102; 16 streams 76.7 -> 77.8). The fused chain has no launch with
+     * work-groups to spare. */
+    const int spread = !fused && n > SPREAD_STREAMS;
+    const pgpu_matrix ada0 = spread ? ada_rows(h, 0, ADA) : h->ada;
     if (!pgpu_head_front(st, &h->cond, conditions, B, norm, norm ? norm + PH_WIDTH : NULL,
                          h->b_cond, tsum, h->silu_split,
                          eos ? &h->eos : NULL, h->b_eos, h->eos_rows, EOS_ROWS, raw, scale,
                          h->noise, h->noise_split, h->status) ||
-        !pgpu_head_mod(st, &h->ada, h->silu_split, B, h->b_ada, h->mod, MOD, &h->input,
+        !pgpu_head_mod(st, &ada0, h->silu_split, B, h->b_ada, h->mod, MOD, &h->input,
                        h->noise_split, h->b_input, h->x, h->status))
         return 0;
-    if (h->fused > 0 || (h->fused < 0 && n <= FUSED_AUTO_STREAMS)) {
+    if (fused) {
         /* x_0 (the input projection) is in xs[0]; block b >= 1 reads
          * x_(b-1) from xs[(b-1) % 2] and block b-1's partials from
          * parts[(b-1) % 2], and writes x_b to xs[b % 2] and its partials to
@@ -408,8 +427,12 @@ static int enqueue_head(PhononFlowHeadDevice *h, size_t n, const float *conditio
         if (cancel && cancel(context))
             return 0;
         const float *mod = h->mod + b * ADA;
-        if (!pgpu_head_mlp_in(st, &h->mlp[b][0], h->x, B, h->norm_w[b], h->norm_b[b], 1e-6f, mod,
-                              MOD, h->b_mlp[b][0], h->first_split, h->status) ||
+        const size_t next = (b + 1) * ADA;
+        const pgpu_matrix ada = ada_rows(h, next, b + 1 < HB ? ADA : FINAL_ADA);
+        const pgpu_matrix *beside = spread ? &ada : NULL;
+        if (!pgpu_head_mlp_in_beside(st, &h->mlp[b][0], h->x, B, h->norm_w[b], h->norm_b[b],
+                                     1e-6f, mod, MOD, h->b_mlp[b][0], h->first_split, beside,
+                                     h->silu_split, h->b_ada + next, h->mod + next, h->status) ||
             !pgpu_gemm_gated(st, &h->mlp[b][1], &first, B, h->b_mlp[b][1], mod + 2 * PH_WIDTH,
                              MOD, h->x, h->x, h->status))
             return 0;

@@ -356,6 +356,33 @@ def test_one_launch_head_equals_the_chain(lib, pkg, streams):
     lib.phonon_flow_head_device_destroy(dev)
 
 
+@pytest.mark.parametrize("streams", [32, 33, 49])
+def test_modulation_beside_the_blocks(lib, pkg, streams):
+    """The chain's frame on both sides of the line from which the adaLN rows run
+    beside the blocks' MLPs, with partial tiles: the bits of the one dataflow
+    launch, which computes them as tasks of its own."""
+    views = pkg.Views()
+    dev = _head_with_frame(lib, pkg, views, 53)
+    stream = lib.phonon_flow_head_device_stream(dev)
+    rng = np.random.default_rng(54)
+    rows = [rng.standard_normal((streams, n)).astype(np.float32) for n in (512, 512, 32)]
+    bufs = [pkg.DeviceBuffer(lib, a.nbytes) for a in rows]
+    for b, a in zip(bufs, rows):
+        b.upload(a)
+    dl, de, dn = (pkg.DeviceBuffer(lib, streams * 4 * n) for n in (32, 1, 512))
+    got = []
+    for one_launch in (0, 1):
+        assert lib.phonon_flow_head_device_set_one_launch(dev, one_launch)
+        assert lib.phonon_flow_head_device_frame(dev, streams, *(b.ptr for b in bufs), 0.6,
+                                                 dl.ptr, de.ptr, dn.ptr)
+        assert lib.phonon_flow_head_device_sync(dev), pkg.last_error(lib)
+        got.append([d.download((streams, n), stream=stream).view(np.uint32)
+                    for d, n in ((dl, 32), (de, 1), (dn, 512))])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    lib.phonon_flow_head_device_destroy(dev)
+
+
 @pytest.mark.parametrize("one_launch", [1, 2])
 def test_one_launch_head_forced_wait_timeout_recovers(lib, pkg, one_launch):
     """A 1 us wait limit, set from the host, makes the one-launch head's
