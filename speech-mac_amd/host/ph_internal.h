@@ -88,9 +88,6 @@ int ph_overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes);
 int ph_batch_enqueue_layers(PhononFlowBatch *batch, size_t first, size_t count,
                             size_t pool_offset, const float *input, float *output,
                             float theta);
-int ph_batch_single_usable(const PhononFlowBatch *b);
-int ph_batch_enqueue_single(PhononFlowBatch *b, size_t position, const int32_t *table_dev,
-                            const float *input, float *output, float theta);
 int ph_batch_set_single(PhononFlowBatch *batch, size_t position, const int32_t *table_dev);
 int ph_batch_set_prefill(PhononFlowBatch *batch, size_t streams, const size_t *first,
                          const size_t *counts, const int32_t *tables_dev);

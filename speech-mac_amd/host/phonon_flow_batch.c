@@ -717,28 +717,6 @@ int ph_batch_enqueue_layers(PhononFlowBatch *b, size_t first, size_t count, size
                          rope);
 }
 
-static int flow_prepare(PhononFlowBatch *b, int prefill);
-static int enqueue_flow(PhononFlowBatch *b, const float *input, float *output, float theta);
-
-/* A whole step of one stream at `position` as one launch, whose tasks give the
- * bits of ph_batch_enqueue_layers (PGPU_FLOW_HANDOFF_MERGE_OUT, set by the
- * caller). A step that follows the batch's last one finds its position and
- * block table in place. */
-int ph_batch_enqueue_single(PhononFlowBatch *b, size_t position, const int32_t *table_dev,
-                            const float *input, float *output, float theta) {
-    const int follows = b->streams == 1 && !b->pre.active && b->host_positions[0] == position;
-    if ((!follows && !ph_batch_set_single(b, position, table_dev)) || !flow_prepare(b, 0) ||
-        !enqueue_flow(b, input, output, theta))
-        return 0;
-    b->host_positions[0]++;
-    return 1;
-}
-
-int ph_batch_single_usable(const PhononFlowBatch *b) {
-    return b->model->layers == (size_t)b->pool->kv.layers && b->model->q8 >= 0 &&
-           b->model->layers <= 63 && b->flow;
-}
-
 /* Stream groups of the step: tiles of 16 streams dealt into `groups` runs.
  * Returns the group count actually used (a group holds >= 1 tile). */
 static size_t group_bounds(const PhononFlowBatch *b, size_t *first, size_t *count) {

@@ -17,7 +17,6 @@
 #include <limits.h>
 #include <math.h>
 #include <pthread.h>
-#include <stdatomic.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -380,31 +379,20 @@ int phonon_linear(const PhononTensorView *weight, const float *input, size_t row
  * one stream at `position`, reading `input` (host [512]) and writing
  * `output` (host [512]); polls `cancel` before every layer and after the
  * last. Copies the appended K/V rows back into the cache's host arrays. */
-static int run_position_beside(int alone, const PhononFlowModel *model, Mirror *m,
-                               PhononKvCache *cache, size_t pool_first, size_t position,
-                               const float *input, float theta, float *output,
-                               PhononCancelPoll cancel, void *context, int *cancelled) {
+static int run_position(const PhononFlowModel *model, Mirror *m, PhononKvCache *cache,
+                        size_t pool_first, size_t position, const float *input, float theta,
+                        float *output, PhononCancelPoll cancel, void *context, int *cancelled) {
     *cancelled = 0;
     const size_t layers = phonon_flow_model_layers(model);
-    if (!m->batch && (!phonon_flow_batch_create(model, m->pool, 1, m->positions, &m->batch) ||
-                      !phonon_flow_batch_set_handoff(m->batch, PGPU_FLOW_HANDOFF_MERGE_OUT)))
+    if (!m->batch && !phonon_flow_batch_create(model, m->pool, 1, m->positions, &m->batch))
         return ph_fail("decode step: batch creation failed");
     PhononFlowBatch *b = m->batch;
     void *s = ph_batch_stream(b);
     float *in = ph_batch_in(b), *out = ph_batch_out(b);
-    if (!ph_batch_bind_model(b, model) ||
+    if (!ph_batch_bind_model(b, model) || !ph_batch_set_single(b, position, m->table_dev) ||
         !pgpu_copy_h2d(s, in, input, PHONON_FLOW_WIDTH * sizeof(float)))
         return ph_fail("decode step: setting up the stream failed");
-    /* One launch for the whole step when it has the GPU to itself and nobody
-     * asks between its layers: its waiting tasks hold most of the work-group
-     * slots, so beside another cache's step the layers go phase by phase,
-     * which leaves room for both. The bits are the same. */
-    const int whole = !cancel && alone && pool_first == 0 && ph_batch_single_usable(b);
-    if (whole && !ph_batch_enqueue_single(b, position, m->table_dev, in, out, theta))
-        return ph_fail("decode step: enqueueing the step failed");
-    if (!whole && !ph_batch_set_single(b, position, m->table_dev))
-        return ph_fail("decode step: setting up the stream failed");
-    for (size_t l = 0; !whole && l < layers; l++) {
+    for (size_t l = 0; l < layers; l++) {
         if (cancel && cancel(context)) {
             *cancelled = 1;
             (void)ph_batch_status(b);
@@ -444,18 +432,6 @@ static int run_position_beside(int alone, const PhononFlowModel *model, Mirror *
         return ph_fail("decode step: non-finite value or uncovered position on the device");
     return ph_all_finite(output, PHONON_FLOW_WIDTH) ||
            ph_fail("decode step: non-finite output");
-}
-
-static atomic_int g_steps; /* steps of any cache under way */
-
-static int run_position(const PhononFlowModel *model, Mirror *m, PhononKvCache *cache,
-                        size_t pool_first, size_t position, const float *input, float theta,
-                        float *output, PhononCancelPoll cancel, void *context, int *cancelled) {
-    const int alone = atomic_fetch_add(&g_steps, 1) == 0;
-    const int ok = run_position_beside(alone, model, m, cache, pool_first, position, input, theta,
-                                       output, cancel, context, cancelled);
-    (void)atomic_fetch_sub(&g_steps, 1);
-    return ok;
 }
 
 /* Prefill of positions [0, length) for the stream of `m`: chunks of up to

@@ -1319,48 +1319,6 @@ def test_forced_wait_timeout_reports_and_recovers(lib, syn, pkg, handoff, stream
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
-def test_dropin_steps_whole_and_by_layers(lib, syn, pkg):
-    """A request's steps as one launch each, mixed with steps that poll a cancel
-    callback (layer by layer), steps beside a prefilled context and a second
-    request in the same cache: outputs and cache rows have the bits of a cache
-    stepped layer by layer throughout."""
-    model = scaled_model(syn, 243, L9)
-    views = pkg.Views()
-    w = views.layers(model)
-    prompt, steps = 5, 6
-    rng = np.random.default_rng(244)
-    xs = rng.standard_normal((2, prompt + steps, 512)).astype(np.float32)
-
-    @pkg.CANCEL_POLL
-    def go_on(_ctx):
-        return 0
-
-    def run(polled):
-        cache, got = Cache(lib, prompt + steps), []
-        for x in xs:
-            lib.phonon_kv_cache_reset(cache.ref())
-            y = np.zeros(512, np.float32)
-            assert lib.phonon_flow_stack_prefill(w, cache.ref(), fp(x), prompt, 10000.0, fp(y))
-            for k in range(steps):
-                y = np.zeros(512, np.float32)
-                row = fp(np.ascontiguousarray(x[prompt + k]))
-                if polled(k):
-                    assert lib.phonon_flow_stack_step_cancel(w, cache.ref(), prompt + k, row,
-                                                             10000.0, fp(y), go_on, None)
-                else:
-                    assert lib.phonon_flow_stack_step(w, cache.ref(), prompt + k, row, 10000.0,
-                                                      fp(y)), pkg.last_error(lib)
-                got.append(y)
-            got.append(cache.keys().copy())
-        cache.destroy()
-        return got
-
-    want = run(lambda k: True)
-    for polled in (lambda k: False, lambda k: k in (1, 2, 4)):
-        for a, b in zip(run(polled), want):
-            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
-
-
 def test_dropins_from_two_threads(lib, syn, pkg):
     """Two host threads drive the reference-signature drop-in
     phonon_flow_stack_step at once on two caches, as concurrent requests on
