@@ -82,6 +82,11 @@ const float *ph_rope_table_long(float theta);
 int ph_all_finite(const float *values, size_t count);
 int ph_overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes);
 
+/* phonon_flow_batch_create with the batch's work on `stream`, which stays the
+ * caller's and outlives the batch (NULL: a stream of the batch's own). */
+int ph_batch_create_on(const PhononFlowModel *model, PhononKvPool *pool, size_t max_streams,
+                       size_t max_positions, void *stream, PhononFlowBatch **batch);
+
 /* Enqueue layers [first, first+count) of the step for the batch's active
  * streams, reading the residual stream from `input` and leaving it in
  * `output` (both dev [streams][512]); pool layer = model layer + pool_offset. */

@@ -39,7 +39,8 @@ struct PhononFlowBatch {
     PhononKvPool *pool;
     size_t max_streams, padded_streams, max_positions, table_len, max_splits, streams;
     size_t splits; /* attention splits of the work being enqueued (<= max_splits) */
-    void *stream;
+    void *stream;     /* the batch's work; its own or its maker's */
+    void *own_stream; /* NULL where the maker's stream is used */
     float *x, *r, *q, *in, *out, *rows;
     uint16_t *xh; /* split fragments of the MLP hidden rows */
     int32_t *positions, *tables;
@@ -427,7 +428,7 @@ void phonon_flow_batch_destroy(PhononFlowBatch *b) {
                     b->fl.rows, b->fl.parts, b->fl.mlp_parts, b->fl.schedule};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
         pgpu_free(bufs[i]);
-    pgpu_stream_destroy(b->stream);
+    pgpu_stream_destroy(b->own_stream);
     free(b->pre.host);
     pgpu_host_free(b->pre.stage);
     free(b->pre.runs_host);
@@ -440,8 +441,8 @@ void phonon_flow_batch_destroy(PhononFlowBatch *b) {
     free(b);
 }
 
-int phonon_flow_batch_create(const PhononFlowModel *model, PhononKvPool *pool,
-                             size_t max_streams, size_t max_positions, PhononFlowBatch **batch) {
+int ph_batch_create_on(const PhononFlowModel *model, PhononKvPool *pool, size_t max_streams,
+                       size_t max_positions, void *stream, PhononFlowBatch **batch) {
     if (!batch)
         return 0;
     *batch = NULL;
@@ -467,10 +468,9 @@ int phonon_flow_batch_create(const PhononFlowModel *model, PhononKvPool *pool,
     b->flow = 1;
     b->fl.place = ph_flow_default_placement(1);
     /* One HIP stream; the side streams of stream groups are made when groups
-     * are asked for (phonon_flow_batch_set_groups), so a batch per request
-     * holds one stream and requests on separate caches spread over the
-     * GPU's hardware queues. */
-    int ok = pgpu_stream_create(&b->stream);
+     * are asked for (phonon_flow_batch_set_groups). */
+    int ok = stream || pgpu_stream_create(&b->own_stream);
+    b->stream = stream ? stream : b->own_stream;
     b->x = pgpu_malloc(rows);
     b->r = pgpu_malloc(rows);
     b->q = pgpu_malloc(rows);
@@ -505,6 +505,11 @@ int phonon_flow_batch_create(const PhononFlowModel *model, PhononKvPool *pool,
     }
     *batch = b;
     return 1;
+}
+
+int phonon_flow_batch_create(const PhononFlowModel *model, PhononKvPool *pool,
+                             size_t max_streams, size_t max_positions, PhononFlowBatch **batch) {
+    return ph_batch_create_on(model, pool, max_streams, max_positions, NULL, batch);
 }
 
 int phonon_flow_batch_set_streams(PhononFlowBatch *b, size_t streams, const size_t *positions,

@@ -25,6 +25,7 @@ typedef struct Mirror {
     size_t capacity, positions, table_len;
     PhononKvPool *pool;
     int32_t *table_host, *table_dev;
+    void *stream; /* both batches' HIP stream: they never run at once (lock) */
     PhononFlowBatch *batch;   /* one stream: decode steps */
     PhononFlowBatch *prefill; /* up to PH_PREFILL_CHUNK positions at once */
     pthread_mutex_t lock;     /* held by a step or prefill of this cache */
@@ -41,6 +42,7 @@ static void mirror_free(Mirror *m) {
         return;
     phonon_flow_batch_destroy(m->batch);
     phonon_flow_batch_destroy(m->prefill);
+    pgpu_stream_destroy(m->stream);
     phonon_kv_pool_destroy(m->pool);
     free(m->table_host);
     if (m->table_dev) {
@@ -49,6 +51,18 @@ static void mirror_free(Mirror *m) {
     }
     pthread_mutex_destroy(&m->lock);
     free(m);
+}
+
+/* The batch at `slot` (made on first use) on the cache's stream. A process
+ * has four hardware queues and streams past that share them, so the decode and
+ * prefill batches of a cache take one stream together: with one each, two
+ * requests held four streams and, beside the null and the library's stream,
+ * their decode steps could come to share a queue (1.6x one request's time for
+ * the two where separate queues take 1.1x). */
+static int mirror_batch(Mirror *m, const PhononFlowModel *model, size_t max_streams,
+                        PhononFlowBatch **slot) {
+    return *slot || ((m->stream || pgpu_stream_create(&m->stream)) &&
+                     ph_batch_create_on(model, m->pool, max_streams, m->positions, m->stream, slot));
 }
 
 static Mirror *mirror_find(const PhononKvCache *cache) {
@@ -384,7 +398,7 @@ static int run_position(const PhononFlowModel *model, Mirror *m, PhononKvCache *
                         float *output, PhononCancelPoll cancel, void *context, int *cancelled) {
     *cancelled = 0;
     const size_t layers = phonon_flow_model_layers(model);
-    if (!m->batch && !phonon_flow_batch_create(model, m->pool, 1, m->positions, &m->batch))
+    if (!mirror_batch(m, model, 1, &m->batch))
         return ph_fail("decode step: batch creation failed");
     PhononFlowBatch *b = m->batch;
     void *s = ph_batch_stream(b);
@@ -446,7 +460,7 @@ static int run_prefill(const PhononFlowModel *model, Mirror *m, PhononKvCache *c
     *cancelled = 0;
     const size_t layers = phonon_flow_model_layers(model);
     const size_t chunk = m->positions < PH_PREFILL_CHUNK ? m->positions : PH_PREFILL_CHUNK;
-    if (!m->prefill && !phonon_flow_batch_create(model, m->pool, chunk, m->positions, &m->prefill))
+    if (!mirror_batch(m, model, chunk, &m->prefill))
         return ph_fail("prefill: batch creation failed");
     PhononFlowBatch *b = m->prefill;
     void *s = ph_batch_stream(b);
