@@ -104,10 +104,42 @@ pgpu_flow_placement ph_flow_default_placement(int rounds) {
      * B = 64 a 16-stream tile's attention is ~640 splits. Swept on MI355X
      * at B = 64 (one split per task) and B = 48, 96, 128, 160 (two), contexts
      * U{1..2048}; a decode step's own placement follows its contexts
-     * (flow_placement in phonon_flow_batch.c). */
+     * (ph_flow_step_placement). */
     const pgpu_flow_placement one = {1.0f, {550.0f, 1000.0f, 1450.0f, 1750.0f}};
     const pgpu_flow_placement two = {2.0f, {1150.0f, 1850.0f, 2550.0f, 3050.0f}};
     return rounds > 1 ? two : one;
+}
+
+/* A tile's QKV, the last of its chain's four phases, belongs just before the
+ * other tiles' attention tasks of the layer run out, for that is when the
+ * tile's next attention can be listed: later and the tile starves, earlier and
+ * the waiting tasks hold slots. The other phases come before it in the
+ * proportion of the times they take. `last` against the others' tasks was swept
+ * on MI355X over 0.58 .. 1.06 of them (one split per task) and 2300 .. 4200
+ * (two), and lies on straight lines between the points below: it is nearly all
+ * of them for few, when the chain takes longer than they do; 0.82 from 2100 on;
+ * from 3700 on less, the chain being long done. It must not jump: at 2022 ..
+ * 2100 others (64 streams, contexts U{1..2048}) a step takes 656 .. 672 us at
+ * 0.82 of them, 666 .. 678 at 0.88 and 695 .. 707 at 0.94, while 1696 (40
+ * streams) take 588 at 0.94 and 609 at 0.82. us per step, contexts U{1..n},
+ * against the fixed offsets above: 24 streams n = 6000 760 / 824; 40, 2048 588 /
+ * 726; 48, 2048 619 / 719; 64, 300 442 / 592; 64, 6000 1402 / 1533; 128, 300 478
+ * / 842; 160, 2048 1575 / 1566; 200, 2048 1870 / 1860. */
+pgpu_flow_placement ph_flow_step_placement(size_t tiles, size_t splits, int rounds) {
+    static const struct {
+        double others, last;
+    } at[] = {{0, 0}, {1700, 1598}, {2100, 1722}, {3700, 3034}, {4200, 3150}, {5600, 4200}};
+    enum { POINTS = sizeof(at) / sizeof(at[0]) };
+    const double others = tiles ? (double)splits * (tiles - 1) / tiles : 0.0;
+    double last = at[POINTS - 1].last;
+    for (int i = 1; i < POINTS; i++)
+        if (others < at[i].others) {
+            last = at[i - 1].last + (at[i].last - at[i - 1].last) * (others - at[i - 1].others) /
+                                        (at[i].others - at[i - 1].others);
+            break;
+        }
+    const float f = (float)last;
+    return (pgpu_flow_placement){(float)rounds, {0.314f * f, 0.571f * f, 0.829f * f, f}};
 }
 
 size_t pgpu_flow_schedule(size_t streams, size_t layers, const size_t *units,

@@ -39,6 +39,9 @@ enum { PH_FLOW_FUSED_DEFAULT_MAX_STREAMS = 2 };
 /* Chain placement of the one-launch step's task list (pgpu_flow_placement):
  * measured on MI355X at B = 64 (ph_flow_schedule.c). */
 pgpu_flow_placement ph_flow_default_placement(int rounds);
+/* That of a decode step of `tiles` 16-stream tiles that lists `splits`
+ * attention splits a layer over all heads, `rounds` to a task. */
+pgpu_flow_placement ph_flow_step_placement(size_t tiles, size_t splits, int rounds);
 
 /* Device selection and the library's own HIP stream (created once). */
 int ph_init(void);

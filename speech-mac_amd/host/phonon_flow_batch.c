@@ -795,23 +795,6 @@ static int flow_rounds(const PhononFlowBatch *b, size_t splits) {
     return splits * PH_HEADS <= PH_FLOW_ONE_ROUND_MAX_SPLITS ? 1 : PGPU_FLOW_ATTN_ROUNDS;
 }
 
-/* Where a decode step lists a tile's chain: its QKV, the last of the four
- * phases, just before the other tiles' attention tasks of the layer run out,
- * for that is when the tile's next attention can be listed; the others before
- * it in the proportion of the times they take. An offset that does not follow
- * the contexts lists the chain too late for short ones (its tile starves) and
- * too early for long ones (waiting tasks hold slots). us per step, contexts
- * U{1..n}, against offsets that were the same for all (550 .. 1750 tasks): 24
- * streams n = 6000 801 / 894; 40, 2048 603 / 744; 48, 2048 636 / 755; 64, 300
- * 462 / 612; 64, 2048 730 / 735; 64, 6000 1511 / 1725; 96, 300 463 / 711; 128,
- * 600 578 / 667. The share of the others' tasks: swept 0.7 .. 1.06; the best
- * lies at 0.94 .. 1 up to 2800 splits and at 0.76 .. 0.88 beyond. */
-static pgpu_flow_placement flow_placement(size_t tiles, size_t splits, int rounds) {
-    const double others = (double)splits * (tiles - 1) / tiles;
-    const float last = (float)(others * (splits <= 2800 ? 0.94 : 0.82));
-    return (pgpu_flow_placement){(float)rounds, {0.314f * last, 0.571f * last, 0.829f * last, last}};
-}
-
 static int flow_usable(const PhononFlowBatch *b, int prefill) {
     if (!b->flow || b->model->q8 < 0 || b->model->layers > 63 || b->streams > 4096)
         return 0;
@@ -944,7 +927,7 @@ static int flow_schedule(PhononFlowBatch *b, int prefill) {
     const pgpu_flow_placement place =
         b->fl.place_set ? b->fl.place
         : prefill       ? ph_flow_default_placement(rounds)
-                        : flow_placement((streams + 15) / 16, splits * PH_HEADS, rounds);
+                        : ph_flow_step_placement((streams + 15) / 16, splits * PH_HEADS, rounds);
     const size_t tasks =
         pgpu_flow_schedule(streams, layers, b->fl.units, &place, flags, NULL, 0);
     if (tasks > b->fl.host_cap) {

@@ -245,3 +245,40 @@ def test_schedule_rejects_unknown_flags(pkg):
     splits = np.ascontiguousarray([1], dtype=np.uintp)
     szp = splits.ctypes.data_as(ctypes.POINTER(ctypes.c_size_t))
     assert lib.pgpu_flow_schedule(1, 1, szp, None, 4, None, 0) == 0
+
+
+def step_offset(lib, tiles, splits, rounds):
+    import speech_mac_amd as pkg
+    fn = lib.ph_flow_step_placement
+    fn.restype, fn.argtypes = pkg.PgpuFlowPlacement, [ctypes.c_size_t, ctypes.c_size_t,
+                                                      ctypes.c_int]
+    p = fn(tiles, splits, rounds)
+    after = list(p.after_us)
+    assert p.unit_us == rounds and after == sorted(after) and after[0] >= 0
+    return after[3]
+
+
+def check_offsets(offset, tiles):
+    """The chain's offset grows with the step's splits without a jump (at most
+    one task per further task of the others), and stays within their number."""
+    at = np.arange(0, 20000, 8)
+    last = np.array([offset(int(n)) for n in at])
+    others = at * (tiles - 1) / tiles
+    assert np.all(last <= others * (1 + 1e-6))
+    step = np.diff(last)
+    assert np.all(step >= -1e-3) and np.all(step <= 8 * (1 + 1e-3))
+
+
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4, 6, 14])
+def test_step_placement_follows_the_splits(pkg, tiles):
+    """64 streams' contexts can list 2800 splits or 2808: neither may have its
+    chains listed far from the other's (a step at 2800 took 708 us where 0.94 of
+    the others' tasks were used up to there and 0.82 beyond, 672 at 0.82)."""
+    lib = pkg.load()
+    check_offsets(lambda n: step_offset(lib, tiles, n, 1), tiles)
+    if tiles > 1:
+        with pytest.raises(AssertionError):
+            check_offsets(lambda n: n * (tiles - 1) / tiles * (0.94 if n <= 2800 else 0.82),
+                          tiles)
+    if tiles == 4:
+        assert abs(step_offset(lib, 4, 2800, 1) / 2100 - 0.82) < 1e-3
