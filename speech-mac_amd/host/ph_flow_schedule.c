@@ -110,6 +110,30 @@ pgpu_flow_placement ph_flow_default_placement(int rounds) {
     return rounds > 1 ? two : one;
 }
 
+/* One while a step is a latency chain, two (fewer, longer attention tasks, which
+ * keep more K/V in flight per work-group slot) once it streams. us per step,
+ * one / two, contexts U{1..n}, splits of a layer over all heads: 16 streams n =
+ * 1000 (400) 410 / 439; 16, 8000 (2232) 880 / 890; 48, 2048 (2008) 611 / 652; 64,
+ * 2048 (2800) 672 / 740; 64, 3000 (3536) 832 / 850; 64, 4000 (4440) 1036 / 997;
+ * 64, 6000 (6296) 1468 / 1400. With more tiles the line lies lower, since what
+ * the other tiles' tasks leave uncovered is shorter: it is drawn at the number of
+ * those (2700, where 3600 splits of four tiles lie). 112, 1000 (2503 of the
+ * others) 640 / 651; 72, 2048 (2803) 823 / 807; 96, 1500 (2900) 849 / 794; 192,
+ * 300 (2816) 676 / 527; 224, 300 (3328) 722 / 576; 128, 1000 (3087) 790 / 732. Up
+ * to two tiles whose contexts fill one task of two splits run those (16 streams,
+ * n = 300: 374 / 365), except the smallest batches. */
+int ph_flow_step_rounds(size_t streams, size_t splits) {
+    enum { ONE_ROUND_STREAMS = 8, ONE_ROUND_SPLITS = 3600, ONE_ROUND_OTHERS = 2700 };
+    const size_t tiles = (streams + 15) / 16, all = splits * PH_HEADS;
+    if (streams <= ONE_ROUND_STREAMS)
+        return 1;
+    if (tiles <= 2 && splits <= 2 * streams)
+        return PGPU_FLOW_ATTN_ROUNDS;
+    return all <= ONE_ROUND_SPLITS && all * (tiles - 1) <= ONE_ROUND_OTHERS * tiles
+               ? 1
+               : PGPU_FLOW_ATTN_ROUNDS;
+}
+
 /* A tile's QKV, the last of its chain's four phases, belongs just before the
  * other tiles' attention tasks of the layer run out, for that is when the
  * tile's next attention can be listed: later and the tile starves, earlier and

@@ -26,10 +26,6 @@ enum { PH_PREFILL_RUN = PGPU_PREFILL_RUN, PH_PREFILL_MIN_GROUPS = 1024 };
  * 1450; B = 192: 1954 vs 2076; B = 224: 2277 vs 2347; B = 256: 2649 vs
  * 2642). */
 enum { PH_FLOW_MIN_TILES = 1, PH_FLOW_MAX_TILES = 14 };
-/* One-launch steps of at most this many streams, or of at most this many
- * attention splits over all heads, run one split per ATTN task (the others
- * PGPU_FLOW_ATTN_ROUNDS; flow_rounds has the measurements). */
-enum { PH_FLOW_ONE_ROUND_MAX_STREAMS = 8, PH_FLOW_ONE_ROUND_MAX_SPLITS = 3600 };
 /* One-launch steps of at most this many streams hand values over as tagged
  * words (phonon_flow_batch_set_handoff). */
 enum { PH_FLOW_TAGGED_MAX_STREAMS = 4 };
@@ -39,7 +35,10 @@ enum { PH_FLOW_FUSED_DEFAULT_MAX_STREAMS = 2 };
 /* Chain placement of the one-launch step's task list (pgpu_flow_placement):
  * measured on MI355X at B = 64 (ph_flow_schedule.c). */
 pgpu_flow_placement ph_flow_default_placement(int rounds);
-/* That of a decode step of `tiles` 16-stream tiles that lists `splits`
+/* Attention splits per ATTN task of a decode step that lists `splits` of them
+ * per layer and head. */
+int ph_flow_step_rounds(size_t streams, size_t splits);
+/* The placement of a decode step of `tiles` 16-stream tiles that lists `splits`
  * attention splits a layer over all heads, `rounds` to a task. */
 pgpu_flow_placement ph_flow_step_placement(size_t tiles, size_t splits, int rounds);
 

@@ -776,25 +776,6 @@ static size_t flow_ml_group(const PhononFlowBatch *b) {
  * than one launch per phase (PH_FLOW_MIN_TILES..PH_FLOW_MAX_TILES 16-stream
  * tiles; prefill and larger batches are attention-bound, where the separate
  * attention kernel streams K/V faster). */
-/* Splits per ATTN task of a step that lists `splits` of them per head: one
- * while a step is a latency chain, two (fewer, longer attention tasks, which
- * keep more K/V in flight per work-group slot) once it streams. us per step,
- * one / two, contexts U{1..n}: 16 streams n = 1000 443 / 469; 24, 2048 538 /
- * 551; 48, 2048 636 / 686; 64, 2048 (3248 splits in all) 730 / 795; 80, 2048
- * (3920) 865 / 814; 64, 6000 (6928) 1585 / 1511. Up to two tiles whose
- * contexts fill one task of two splits run those (12 streams, n = 300: 369 /
- * 364), except the smallest batches. */
-static int flow_rounds(const PhononFlowBatch *b, size_t splits) {
-    if (b->fl.rounds_set)
-        return b->fl.rounds_set;
-    const size_t tiles = (b->streams + 15) / 16;
-    if (b->streams <= PH_FLOW_ONE_ROUND_MAX_STREAMS)
-        return 1;
-    if (tiles <= 2 && splits <= 2 * b->streams)
-        return PGPU_FLOW_ATTN_ROUNDS;
-    return splits * PH_HEADS <= PH_FLOW_ONE_ROUND_MAX_SPLITS ? 1 : PGPU_FLOW_ATTN_ROUNDS;
-}
-
 static int flow_usable(const PhononFlowBatch *b, int prefill) {
     if (!b->flow || b->model->q8 < 0 || b->model->layers > 63 || b->streams > 4096)
         return 0;
@@ -918,7 +899,7 @@ static int flow_schedule(PhononFlowBatch *b, int prefill) {
         b->fl.cover[s] = need < b->max_splits ? need : b->max_splits;
         splits += b->fl.cover[s];
     }
-    const int rounds = flow_rounds(b, splits);
+    const int rounds = b->fl.rounds_set ? b->fl.rounds_set : ph_flow_step_rounds(streams, splits);
     splits = 0;
     for (size_t s = 0; s < streams; s++) {
         b->fl.units[s] = (b->fl.cover[s] + rounds - 1) / rounds;

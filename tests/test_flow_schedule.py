@@ -282,3 +282,15 @@ def test_step_placement_follows_the_splits(pkg, tiles):
                           tiles)
     if tiles == 4:
         assert abs(step_offset(lib, 4, 2800, 1) / 2100 - 0.82) < 1e-3
+
+
+@pytest.mark.parametrize("streams,splits,rounds", [
+    (8, 2000, 1), (9, 18, 2), (9, 19, 1), (32, 64, 2), (32, 65, 1), (33, 66, 1), (16, 450, 1),
+    (16, 451, 2), (64, 450, 1), (64, 451, 2), (128, 385, 1), (128, 386, 2), (192, 384, 2),
+    (224, 448, 2), (160, 375, 1), (160, 376, 2)])
+def test_step_rounds_on_both_sides(pkg, streams, splits, rounds):
+    """One split per attention task or two, on both sides of each line: many
+    streams of short contexts run two (224 streams of up to 300 positions: 576 us
+    a step, 722 with one)."""
+    lib = pkg.load()
+    assert lib.ph_flow_step_rounds(ctypes.c_size_t(streams), ctypes.c_size_t(splits)) == rounds
