@@ -150,9 +150,19 @@ int ph_flow_step_rounds(size_t streams, size_t splits) {
  * 726; 48, 2048 619 / 719; 64, 300 442 / 592; 64, 6000 1402 / 1533; 128, 300 478
  * / 842; 160, 2048 1575 / 1566; 200, 2048 1870 / 1860. */
 pgpu_flow_placement ph_flow_step_placement(size_t tiles, size_t splits, int rounds) {
-    static const struct {
+    /* More than eight tiles leave "nearly all" earlier: 224 streams, n = 100, 578
+     * at 0.94 of 1664 others, 481 at 0.82 (fixed offsets 535); 176, 100 484 at 0.94
+     * of 1280, 449 at 0.86; 144, 100 434 at 0.94 of 1024, 480 at 0.86; but 128, 240
+     * 472 at 0.82 of 1792, 452 at 0.9. */
+    const int many = tiles > 8;
+    const struct {
         double others, last;
-    } at[] = {{0, 0}, {1700, 1598}, {2100, 1722}, {3700, 3034}, {4200, 3150}, {5600, 4200}};
+    } at[] = {{0, 0},
+              {many ? 1024 : 1700, many ? 0.94 * 1024 : 0.94 * 1700},
+              {many ? 1536 : 2100, many ? 0.82 * 1536 : 0.82 * 2100},
+              {3700, 0.82 * 3700},
+              {4200, 0.75 * 4200},
+              {5600, 0.75 * 5600}};
     enum { POINTS = sizeof(at) / sizeof(at[0]) };
     const double others = tiles ? (double)splits * (tiles - 1) / tiles : 0.0;
     double last = at[POINTS - 1].last;
