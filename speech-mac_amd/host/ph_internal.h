@@ -15,6 +15,9 @@ enum { PH_MAX_GROUPS = 4, PH_DEFAULT_GROUPS = 1 };
 /* The one-launch step keeps this many positions of headroom in its task
  * schedule (and captured graph) before it has to rebuild them. */
 enum { PH_FLOW_HEADROOM = 256 };
+/* Steps between calls of phonon_flow_batch_set_streams, while the contexts are
+ * much shorter than the task list was made for, after which it is rebuilt. */
+enum { PH_FLOW_LOOSE_STEPS = 4 };
 /* Batched prefill attention (pgpu_prefill_attention): up to PH_PREFILL_RUN
  * consecutive positions per work entry, fewer while the entries would give
  * under PH_PREFILL_MIN_GROUPS work-groups (one per head per entry). */

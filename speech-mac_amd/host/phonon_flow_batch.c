@@ -85,6 +85,9 @@ struct PhononFlowBatch {
         int rounds;                 /* splits per ATTN task the schedule was built for */
         int rounds_set;             /* 0: by batch and contexts, else the caller's choice */
         int rounds_for;             /* rounds_set when the schedule was built */
+        size_t listed;              /* the sum of cover */
+        unsigned ran, loose;        /* flow_loosen */
+        int dropped;                /* by it */
         int place_set;              /* the caller set the placement */
         size_t streams, layers;     /* what the schedule was built for (0: none) */
         int prefill, fused;
@@ -512,6 +515,33 @@ int phonon_flow_batch_create(const PhononFlowModel *model, PhononKvPool *pool,
     return ph_batch_create_on(model, pool, max_streams, max_positions, NULL, batch);
 }
 
+/* Splits that stream s lists: those of its context PH_FLOW_HEADROOM positions
+ * ahead. */
+static size_t flow_need(const PhononFlowBatch *b, size_t s) {
+    const size_t need = (b->host_positions[s] + PH_FLOW_HEADROOM + PH_SPLIT_KEYS) / PH_SPLIT_KEYS;
+    return need < b->max_splits ? need : b->max_splits;
+}
+
+/* Drops the one-launch step's task list when the contexts just set are so much
+ * shorter than those it was made for (other requests in the same slots) that its
+ * splits per task and its chains' places (ph_flow_step_placement) are another
+ * batch's: less than 7/8 of the listed splits, which at steps between two calls
+ * as here (`ran`) have added up to PH_FLOW_LOOSE_STEPS while that held. So a
+ * program that sets long and short contexts in turn for a step each does not pay
+ * for a new list every time (about 0.1 ms). us per step on the long contexts' list
+ * / on a new one: 200 streams U{1..4000} -> U{1..300} 1054 / 554; 160, 4000 -> 600
+ * 1042 / 671; 96, 4000 -> 300 532 / 462; 64 and fewer within 1%. */
+static void flow_loosen(PhononFlowBatch *b) {
+    size_t splits = 0;
+    for (size_t s = 0; s < b->streams; s++)
+        splits += flow_need(b, s);
+    if (b->fl.streams != b->streams || b->fl.prefill || splits * 8 >= b->fl.listed * 7)
+        b->fl.loose = 0;
+    else if ((b->fl.loose += b->fl.ran) >= PH_FLOW_LOOSE_STEPS)
+        b->fl.dropped = 1;
+    b->fl.ran = 0;
+}
+
 int phonon_flow_batch_set_streams(PhononFlowBatch *b, size_t streams, const size_t *positions,
                                   const int32_t *tables, size_t table_len) {
     if (!b || !streams || streams > b->max_streams || !positions || !tables ||
@@ -537,6 +567,7 @@ int phonon_flow_batch_set_streams(PhononFlowBatch *b, size_t streams, const size
     b->pos_lag = 0;
     b->streams = streams;
     b->pre.active = 0;
+    flow_loosen(b);
     return 1;
 }
 
@@ -878,27 +909,29 @@ static int flow_mode(const PhononFlowBatch *b, int prefill) {
 }
 
 /* Rebuilds (and uploads) the step's task list (pgpu_flow_schedule) when the
- * streams, the layers or a context outgrow it. A stream lists the splits of
- * its context PH_FLOW_HEADROOM positions ahead; tasks past its live context
- * end at once. */
+ * streams, the layers or a context outgrow it, or flow_loosen dropped it. Tasks
+ * past a live context end at once. */
 static int flow_schedule(PhononFlowBatch *b, int prefill) {
     const size_t streams = b->streams, layers = b->model->layers;
     const int fused = flow_mode(b, prefill) == PGPU_FLOW_HANDOFF_FUSED_MLP;
     const int flags = (prefill ? PGPU_FLOW_SCHEDULE_PREFILL : 0) |
                       (fused ? PGPU_FLOW_SCHEDULE_FUSED_MLP : 0);
-    int valid = b->fl.streams == streams && b->fl.layers == layers && b->fl.prefill == prefill &&
+    int valid = !b->fl.dropped && b->fl.streams == streams && b->fl.layers == layers &&
+                b->fl.prefill == prefill &&
                 b->fl.rounds_for == b->fl.rounds_set && b->fl.fused == fused;
     for (size_t s = 0; valid && s < streams; s++)
         valid = (b->host_positions[s] + PH_SPLIT_KEYS) / PH_SPLIT_KEYS <= b->fl.cover[s];
     if (valid)
         return 1;
     b->fl.streams = 0; /* no valid schedule until the new one is uploaded */
+    b->fl.loose = 0;
+    b->fl.dropped = 0;
     size_t splits = 0;
     for (size_t s = 0; s < streams; s++) {
-        size_t need = (b->host_positions[s] + PH_FLOW_HEADROOM + PH_SPLIT_KEYS) / PH_SPLIT_KEYS;
-        b->fl.cover[s] = need < b->max_splits ? need : b->max_splits;
+        b->fl.cover[s] = flow_need(b, s);
         splits += b->fl.cover[s];
     }
+    b->fl.listed = splits;
     const int rounds = b->fl.rounds_set ? b->fl.rounds_set : ph_flow_step_rounds(streams, splits);
     splits = 0;
     for (size_t s = 0; s < streams; s++) {
@@ -1025,6 +1058,7 @@ static int enqueue_flow(PhononFlowBatch *b, const float *input, float *output, f
         return 0;
     b->fl.parity = 1 - b->fl.parity;
     b->fl.tag++;
+    b->fl.ran++;
     b->pos_lag++;
     return 1;
 }

@@ -1110,6 +1110,60 @@ def test_schedule_follows_the_contexts(lib, syn, pkg, streams, high):
     assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[3])
 
 
+def test_schedule_follows_contexts_that_shrink(lib, syn, pkg):
+    """Long contexts replaced by short ones in the same batch: after a few steps
+    between two calls that set them, the next step has the task list of a batch
+    that never held the long ones, and its bits; set in turn for one step each,
+    the list stays the long ones'."""
+    layers, streams, high = 2, 40, 4000
+    model, views = scaled_model(syn, 185, layers), pkg.Views()
+    w = views.layers(model)
+    rng = np.random.default_rng(189)
+    long, short = (rng.integers(1, n, streams).astype(np.uintp) for n in (high, 200))
+    table_len = -(-(high + 8) // 16)
+    x = rng.standard_normal((streams, 512)).astype(np.float32)
+
+    def batch():
+        bt = Batch(lib, w, layers, streams, 16 * table_len, streams * table_len)
+        assert lib.phonon_kv_pool_fill_normal(bt.pool, 190)
+        ids = np.zeros(streams * table_len, np.int32)
+        assert lib.phonon_kv_pool_alloc(bt.pool, ids.size, i32p(ids))
+        return bt, np.ascontiguousarray(ids.reshape(streams, table_len))
+
+    def run(bt, tables, lengths, steps):
+        assert lib.phonon_flow_batch_set_streams(
+            bt.batch, streams, lengths.ctypes.data_as(ctypes.POINTER(ctypes.c_size_t)),
+            i32p(tables), table_len)
+        y = np.zeros((streams, 512), np.float32)
+        for _ in range(steps):
+            assert lib.phonon_flow_batch_step(bt.batch, fp(x), 10000.0, fp(y)), pkg.last_error(lib)
+        return y
+
+    def tasks(bt):
+        n = lib.phonon_flow_batch_schedule(bt.batch, None, 0)
+        out = np.zeros(n, np.uint32)
+        u32 = out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))
+        assert lib.phonon_flow_batch_schedule(bt.batch, u32, n) == n
+        return out
+
+    bt, tables = batch()
+    expected = run(bt, tables, short, 1)
+    fresh = tasks(bt)
+    bt.close()
+    bt, tables = batch()
+    run(bt, tables, long, 1)
+    whole = tasks(bt)
+    assert whole.size > fresh.size
+    for lengths in (short, long, short, long):
+        run(bt, tables, lengths, 1)
+        assert np.array_equal(tasks(bt), whole)
+    run(bt, tables, long, 4)
+    got = run(bt, tables, short, 1)
+    assert np.array_equal(tasks(bt), fresh)
+    assert np.array_equal(got.view(np.uint32), expected.view(np.uint32))
+    bt.close()
+
+
 @pytest.mark.parametrize("streams", [1, 2, 4])
 def test_fused_mlp_step_vs_oracle(lib, oracle, oracle_mod, syn, pkg, streams):
     """The fused-MLP hand-off (mode 4: no MLP-out phase; each MLP-in task's
