@@ -50,7 +50,8 @@ size_t phonon_mimi_positions(const PhononMimiState *state);
 /* src/phonon_mimi.h:37-42: row-major [frames,32] -> [frames*16,512]; capacity
  * in feature rows; input and output must not overlap. On a processing
  * failure the state is unusable until reset (the output may hold a partial
- * prefix); invalid arguments leave it untouched. At most 8192 frames per
+ * prefix); invalid arguments, or no memory for the call's intermediates, leave
+ * it untouched. At most 8192 frames per
  * request. */
 int phonon_mimi_process(PhononMimiState *state, const float *latents, size_t frames,
                         float *features, size_t capacity);

@@ -28,7 +28,8 @@ void phonon_pcm_state_reset(PhononPCMState *state);
 size_t phonon_pcm_samples(const PhononPCMState *state);
 /* src/phonon_pcm.h:20-32: [frames,32] -> frames*1920 samples into raw (and
  * final, which may be NULL or raw, else must not overlap); capacities count
- * samples; at most 8192 frames per request. */
+ * samples; at most 8192 frames per request. Invalid arguments, or no memory for
+ * the call's intermediates, leave the state untouched. */
 int phonon_pcm_process(PhononPCMState *state, const float *latents, size_t frames, float *raw,
                        size_t raw_capacity, float *final, size_t final_capacity);
 /* src/phonon_pcm.h:33-36. */
