@@ -1,9 +1,11 @@
 """What the audio decoder's calls allocate (host/phonon_audio.c on stub_device.c,
-without a GPU): everything is given back with the last model and state, and a call
-that finds no memory is refused with its request unharmed."""
+without a GPU): nothing once as many calls as ever have run at the same moment,
+everything given back with the last model and state, and a call that finds no
+memory refused with its request unharmed."""
 import ctypes
 import os
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -11,6 +13,7 @@ import pytest
 import helpers
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CALLS = 8
 
 
 @pytest.fixture(scope="module")
@@ -44,13 +47,25 @@ class Request:
         return self.ok
 
 
+def together(lib, requests, frames):
+    """One call of each request, all of them in flight at the same moment."""
+    lib.stub_wait_for(len(requests))
+    threads = [threading.Thread(target=r.call, args=(frames,)) for r in requests]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(30)
+    lib.stub_wait_for(0)
+    assert all(r.ok == 1 for r in requests)
+
+
 @pytest.fixture
 def model(host, pkg):
     views = pkg.Views()
     before = host.stub_held()
     _, handle = helpers.pcm_model(host, pkg, views, helpers.mimi_identity_model(route_only=True),
                                   helpers.pcm_scalar_convs())
-    requests = [Request(host, handle)]
+    requests = [Request(host, handle) for _ in range(CALLS)]
     yield requests, handle
     for r in requests:
         host.phonon_pcm_state_destroy(r.h)
@@ -60,14 +75,53 @@ def model(host, pkg):
     assert host.stub_held() - before in (0, 8192 * 16 * 64 * 4 + 1)
 
 
+def test_calls_in_step_allocate_once(host, model):
+    requests, _ = model
+    for frames in (1, 9):
+        together(host, requests, frames)
+        made, released = host.stub_made(), host.stub_released()
+        for _ in range(3):
+            together(host, requests, frames)
+        assert (host.stub_made(), host.stub_released()) == (made, released)
+
+
+def test_a_frame_at_a_time_holds_little(host, model):
+    """Eight states a frame at a time hold 8 x 11.5 MB of intermediates and 8 x 0.13
+    of pinned memory; a block for 64 frames alone is 92."""
+    requests, _ = model
+    before = host.stub_held()
+    together(host, requests, 1)
+    assert 0 < host.stub_held() - before < CALLS * 12_000_000
+
+
+def test_states_that_go_give_theirs_back(host, model):
+    requests, handle = model
+    held = host.stub_held()
+    requests.append(Request(host, handle))
+    state = host.stub_held() - held
+    together(host, requests, 1)
+    full = host.stub_held()
+    while len(requests) > 1:
+        host.phonon_pcm_state_destroy(requests.pop().h)
+    given = full - host.stub_held() - CALLS * state
+    assert given >= (CALLS - 2) * 11_500_000
+    # Requests that come and go one after another allocate no intermediates.
+    assert requests[0].call(1) == 1
+    held = host.stub_held()
+    r = Request(host, handle)
+    assert r.call(1) == 1 and host.stub_held() - held == state
+    host.phonon_pcm_state_destroy(r.h)
+
+
 def test_a_call_without_memory_leaves_its_request_usable(host, model):
     requests, _ = model
     r = requests[0]
+    assert r.call(2) == 1 and host.phonon_pcm_samples(r.h) == 2 * 1920
     host.stub_fail(1)
-    assert r.call(40) == 0
+    assert r.call(40) == 0  # no block of that size yet
     host.stub_fail(0)
-    assert host.phonon_pcm_samples(r.h) == 0
-    assert r.call(40) == 1 and host.phonon_pcm_samples(r.h) == 40 * 1920
+    assert host.phonon_pcm_samples(r.h) == 2 * 1920
+    assert r.call(40) == 1 and host.phonon_pcm_samples(r.h) == 42 * 1920
 
 
 def test_a_mimi_call_without_memory_leaves_its_state_usable(host, pkg):

@@ -459,9 +459,9 @@ def test_pcm_tile_shapes_and_passes(lib, pkg, oracle, oracle_mod, counts):
 
 
 def test_pcm_calls_from_several_threads(lib, pkg):
-    """Four states, each in a thread of its own, more calls at once than the
-    library keeps staging memory for: every request has the bits of the same
-    request alone."""
+    """Four states, each in a thread of its own, with calls of one and of two
+    passes at the same time: every request has the bits of the same request
+    alone."""
     import threading
     views = pkg.Views()
     mimi_w, convs = random_mimi(921), random_pcm_convs(922)
