@@ -1205,7 +1205,13 @@ static size_t pair_count(size_t streams, const size_t *counts, size_t run) {
  * than half the CUs (8 per pair). A 12-layer call, us, short against long
  * runs: 3 prompts / 611 positions 797 / 947, 4 / 1024 814 / 898, 6 / 1613 over
  * contexts of up to 900 1364 / 1455 (14 pairs); 8 / 2048 1305 / 1293 (16);
- * 16 / 4096 2250 / 2083; 10 / 3523 over contexts of up to 1100 2768 / 2592.
+ * 16 / 4096 2250 / 2083; 10 / 3523 over contexts of up to 1100 2768 / 2592. A
+ * long context does not move the line, though every run of 16 reads it again: one
+ * prompt of 512 after 4000 positions 1766 / 3161, of 1800 (15 pairs) after 6300
+ * 5519 / 5884; 4 to 14 ragged ones of 12 to 15 pairs over contexts of up to 4000
+ * gained 2 to 54%. The one side that loses, up to 8%, is equal prompts at equal
+ * contexts whose runs of 16 are more than 96 (three work-groups on each CU): 15 of
+ * 100 after 6300 5343 / 4930, where 15 of 96 take 4126 / 4854.
  * Without fp16 weights (pgpu_prefill_attention_mfma either way): at most 512
  * positions, so that a short prompt spreads over more work-groups. */
 enum { PH_PREFILL_SHORT_RUN = 16, PH_PREFILL_MIN_PAIRS = 16, PH_PREFILL_SHORT_TOTAL = 512 };
