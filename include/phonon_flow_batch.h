@@ -103,11 +103,17 @@ int phonon_flow_batch_prefill_device(PhononFlowBatch *batch, size_t streams, con
  * attention and merge, so every output row has the bits of single steps;
  * 0 (default) and 2 fast: where a layer's matrices are Q8, the projections
  * on the fp16 matrix cores with two fp16 split terms of each activation (22
- * significant bits), and a causal attention that loads each 64-key chunk
- * once per run of 64 positions: 0 on the fp16 matrix cores with the same
- * two-term splits of q, K, V and the probabilities, 2 with one lane per
- * query on the vector units (fp32). The fast modes stay within 1e-4 of the
- * exact one (normwise per row). */
+ * significant bits), and a causal attention. 2: one lane per query on the
+ * vector units (fp32). 0: on the matrix cores, in one of two forms that the
+ * call's prompts choose together. Many of them: each 64-key chunk is loaded once
+ * per run of 64 positions, on the 16-bit matrix cores with split terms of q, K, V
+ * and the probabilities (three bf16 of q and K, two fp16 of the others, so a V of
+ * 65504 or more is reported as non-finite). Fewer than 16 pairs of such runs (a
+ * prompt of n positions has ceil(ceil(n / 64) / 2)): runs of 16 positions with
+ * fp32 products. The fast modes stay within 1e-4 of the exact one (normwise per
+ * row). With 1 and 2 a prompt's rows and K/V have the same bits whatever else is in
+ * the call; with 0 they may differ, within those bounds, between a call of few
+ * prompts and one of many. */
 int phonon_flow_batch_set_prefill_exact(PhononFlowBatch *batch, int exact);
 /* One-launch step: a task that has waited this many microseconds for its
  * inputs (at most 10 s) gives up, sets status bit 2 (value 4) and makes

@@ -867,11 +867,10 @@ def test_batched_prefill_equals_single_steps(lib, syn, pkg, mode, exact):
 @pytest.mark.parametrize("counts,first", [([256, 256], [0, 0]), ([200, 57, 255], [0, 40, 0]),
                                           ([257, 256], [0, 0])])
 def test_fast_prefill_around_the_short_prompt_path(lib, syn, pkg, counts, first):
-    """The fast prefill of 512 positions in one call (the short-prompt path:
-    64 x 32 projection tiles, attention runs of 16 positions; with ragged
-    counts and a continued context) and of 513 (the large tiles, runs of
-    64) against the exact prefill of the same call, which gives the bits of
-    single decode steps: every output row within 1e-4 normwise."""
+    """The fast prefill of 512 positions in one call (with ragged counts and a
+    continued context) and of 513 against the exact prefill of the same call,
+    which gives the bits of single decode steps: every output row within 1e-4
+    normwise."""
     layers = 2
     model = scaled_model(syn, 191, layers)
     w = pkg.Views().layers(model)
@@ -966,6 +965,53 @@ def test_fast_prefill_tiles_and_runs(lib, syn, pkg, counts, first):
     worst = max(helpers.normwise(b, a) for a, b in zip(outs[0], outs[1]))
     print(f"fast prefill of {counts} at {first} vs exact: max normwise {worst:.3g}", flush=True)
     assert worst <= 1e-4
+
+
+@pytest.mark.parametrize("exact", [0, 1, 2])
+def test_prefill_of_a_prompt_alone_and_beside_others(lib, syn, pkg, exact):
+    """One prompt of 200 positions after 40 held, prefilled alone (runs of 16 on
+    fp32 products in the default mode) and in one call with 16 other prompts (20
+    pairs of long runs, 16-bit products): the same bits with the exact mode and
+    with one lane per query. The default's two forms are each within 1e-4 of the
+    exact mode, so within 2e-4 of each other."""
+    layers, mine, held = 2, 200, 40
+    model, views = scaled_model(syn, 196, layers), pkg.Views()
+    w = views.layers(model)
+    rng = np.random.default_rng(197)
+    ctx = rng.standard_normal((2, layers, held, 512)).astype(np.float32)
+    others = [int(n) for n in rng.integers(20, 64, 16)]
+    x = rng.standard_normal((mine + sum(others), 512)).astype(np.float32)
+    szp = ctypes.POINTER(ctypes.c_size_t)
+    table_len = 16
+    got = []
+    for counts in ([mine], [mine] + others):
+        n, total = len(counts), sum(counts)
+        bt = Batch(lib, w, layers, total, 16 * table_len, n * table_len)
+        ids = np.zeros(n * table_len, np.int32)
+        assert lib.phonon_kv_pool_alloc(bt.pool, ids.size, i32p(ids))
+        tables = np.ascontiguousarray(ids.reshape(n, table_len))
+        assert lib.phonon_kv_pool_write(bt.pool, i32p(tables[0]), table_len, 0, held, fp(ctx[0]),
+                                        fp(ctx[1]), held)
+        f, c = np.zeros(n, np.uintp), np.array(counts, np.uintp)
+        f[0] = held
+        assert lib.phonon_flow_batch_set_prefill_exact(bt.batch, exact)
+        din, dout = (pkg.DeviceBuffer(lib, total * 2048) for _ in range(2))
+        din.upload(x[:total])
+        assert lib.phonon_flow_batch_prefill_device(bt.batch, n, f.ctypes.data_as(szp),
+                                                    c.ctypes.data_as(szp), i32p(tables),
+                                                    table_len, din.ptr, 10000.0, dout.ptr), \
+            pkg.last_error(lib)
+        assert lib.phonon_flow_batch_sync(bt.batch)
+        got.append(dout.download((total, 512))[:mine])
+        din.free()
+        dout.free()
+        bt.close()
+    if exact:
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    else:
+        worst = max(helpers.normwise(b, a) for a, b in zip(*got))
+        print(f"fast prefill alone vs beside 16 prompts: max normwise {worst:.3g}", flush=True)
+        assert worst <= 2e-4
 
 
 def test_prefill_calls_enqueued_back_to_back(lib, syn, pkg):
