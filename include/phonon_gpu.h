@@ -330,7 +330,9 @@ int pgpu_prefill_attention(void *stream, const float *q, const pgpu_paged_kv *kv
                            int *status);
 /* -- audio decoder (pgpu_audio.hip). Positions are rows of row-major
  * [positions][channels] device arrays; every kernel covers all positions of
- * a call at once, taking earlier positions from the caller's history. -- */
+ * a call at once, taking earlier positions from the caller's history. The library's
+ * own decoder runs other forms of the Mimi steps (its rows as split terms); the
+ * three below are for callers with fp32 rows of their own. -- */
 /* Mimi input of `frames` latent frames ([frames][32]): the 512 x 32
  * projection (fp32 [512][32]) and the depthwise upsample (fp32 [512][32]:
  * taps 0..15 current frame, 16..31 previous frame) into hidden

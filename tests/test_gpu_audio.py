@@ -117,10 +117,10 @@ def test_mimi_synthetic_ring_and_scales(lib, pkg):
 
 
 def test_mimi_random_weights_ring_wrap_against_oracle(lib, pkg, oracle, oracle_mod):
-    """70 frames = 1120 positions: past the 1024-row device ring, past one
-    32-frame device pass, and every row against the oracle; then the same
-    request in uneven calls, bit for bit."""
-    frames = 70
+    """96 frames = 1536 positions: past the 1280-row device ring (80 frames) and
+    one 64-frame device pass, and every row against the oracle; then the same
+    request in uneven calls, one of them over the wrap, bit for bit."""
+    frames = 96
     w = random_mimi(811)
     x = np.random.default_rng(812).standard_normal((frames, 32)).astype(np.float32)
     om = oracle_mod.MimiOracle(oracle, w)
@@ -138,7 +138,7 @@ def test_mimi_random_weights_ring_wrap_against_oracle(lib, pkg, oracle, oracle_m
     assert err <= TOL and max(rows) <= TOL
     lib.phonon_mimi_state_reset(m.h)
     parts, off = [], 0
-    for count in (1, 33, 5, 31):
+    for count in (1, 33, 44, 5, 13):
         ok, y = m.process(x[off:off + count])
         assert ok == 1
         parts.append(y)
@@ -177,6 +177,63 @@ def test_mimi_attention_windows(lib, pkg, first, frames, context, ring):
             e = np.exp(score - score.max())
             exp[r, d] = e @ kv[1][at, d].astype(np.float64) / e.sum()
     assert normwise(got, exp) <= 1e-5
+
+
+def upload(pkg, lib, a):
+    b = pkg.DeviceBuffer(lib, a.nbytes)
+    b.upload(a)
+    return b
+
+
+@pytest.mark.parametrize("frames", [1, 2, 5])
+def test_mimi_input_rows(lib, pkg, frames):
+    """Projection and depthwise upsample of a call's frames, the frame before them
+    taken from `previous` and the last one left there, against float64: sums of 32
+    and 2 terms in fp32, 1e-6 of the largest result."""
+    rng = np.random.default_rng(frames)
+    lat, proj, up, prev = (rng.standard_normal(n).astype(np.float32)
+                           for n in ((frames, 32), (512, 32), (512, 32), (512,)))
+    d = [upload(pkg, lib, a) for a in (lat, proj, up, prev)]
+    hidden = upload(pkg, lib, np.full((16 * frames, 512), np.nan, np.float32))
+    status = upload(pkg, lib, np.zeros(1, np.int32))
+    assert lib.pgpu_mimi_input(None, d[0].ptr, frames, d[1].ptr, d[2].ptr, d[3].ptr, hidden.ptr,
+                               status.ptr) == 1
+    cur = lat.astype(np.float64) @ proj.astype(np.float64).T
+    before = np.concatenate([prev[None].astype(np.float64), cur[:-1]])
+    exp = before[:, None] * up.T[16:].astype(np.float64) + cur[:, None] * up.T[:16]
+    got = hidden.download((frames, 16, 512), np.float32)
+    assert status.download((1,), np.int32)[0] == 0
+    assert np.max(np.abs(got - exp)) <= 1e-6 * np.max(np.abs(exp))
+    left = d[3].download((512,), np.float32)
+    assert np.max(np.abs(left - cur[-1])) <= 1e-6 * np.max(np.abs(cur))
+
+
+def test_mimi_rope_store_over_the_wrap(lib, pkg):
+    """RoPE of q in place and of k into its ring slot, v beside it, over the ring's
+    end: the fp32 products and sums of the formula, slots of other positions left."""
+    rows, first, ring = 48, 40, 64
+    rng = np.random.default_rng(40)
+    qkv = rng.standard_normal((rows, 1536)).astype(np.float32)
+    angle = rng.uniform(0, 6.28, (first + rows, 32))
+    rope = np.stack([np.cos(angle), np.sin(angle)], -1).astype(np.float32)
+    old = rng.standard_normal((2, ring, 512)).astype(np.float32)
+    dq, dr = upload(pkg, lib, qkv), upload(pkg, lib, rope)
+    dk, dv = upload(pkg, lib, old[0]), upload(pkg, lib, old[1])
+    assert lib.pgpu_mimi_rope_store(None, dq.ptr, rows, first, dr.ptr, first + rows, dk.ptr,
+                                    dv.ptr, ring) == 1
+    cs = np.tile(rope[first:first + rows, None], (1, 8, 1, 1))  # [row][head][pair]
+
+    def turned(x):
+        x = x.reshape(rows, 8, 32, 2)
+        return np.stack([x[..., 0] * cs[..., 0] - x[..., 1] * cs[..., 1],
+                         x[..., 0] * cs[..., 1] + x[..., 1] * cs[..., 0]], -1).reshape(rows, 512)
+
+    slots = (first + np.arange(rows)) % ring
+    k, v = old[0].copy(), old[1].copy()
+    k[slots], v[slots] = turned(qkv[:, 512:1024]), qkv[:, 1024:]
+    assert np.array_equal(dq.download((rows, 1536), np.float32)[:, :512], turned(qkv[:, :512]))
+    assert np.array_equal(dk.download((ring, 512), np.float32), k)
+    assert np.array_equal(dv.download((ring, 512), np.float32), v)
 
 
 def test_mimi_rejects_bad_requests(lib, pkg):
@@ -387,10 +444,11 @@ def test_pcm_scalar_graph(lib, pkg):
 
 
 def test_pcm_random_weights_against_oracle(lib, pkg, oracle, oracle_mod):
-    """Random weights through the whole decoder: 35 frames (one full 32-frame
-    device pass and a partial one) against the oracle, then the same frames
-    in uneven calls, bit for bit."""
-    frames = 35
+    """Random weights through the whole decoder: 66 frames in one call (two
+    device passes, the second one's convolutions and attention reading what the
+    first left) against the oracle, then the same frames in uneven calls, bit
+    for bit."""
+    frames = 66
     mimi_w = random_mimi(901)
     convs = random_pcm_convs(902)
     x = np.random.default_rng(903).standard_normal((frames, 32)).astype(np.float32)
@@ -412,7 +470,7 @@ def test_pcm_random_weights_against_oracle(lib, pkg, oracle, oracle_mod):
     assert err <= TOL and frame_err <= TOL
     lib.phonon_pcm_state_reset(p.h)
     parts, off = [], 0
-    for count in (2, 31, 2):
+    for count in (2, 31, 33):
         ok, r, _ = p.process(x[off:off + count])
         assert ok == 1
         parts.append(r)
@@ -426,8 +484,9 @@ def test_pcm_random_weights_against_oracle(lib, pkg, oracle, oracle_mod):
 def test_pcm_tile_shapes_and_passes(lib, pkg, oracle, oracle_mod, counts):
     """Calls whose passes take each tile shape of the convolutions (from one
     frame's 16 positions to a full pass, with remainders), calls of two and three
-    passes, the ring's wrap (past 128 frames) and requests after a reset: the bits
-    of one frame at a time, whose first frames are the oracle's. The state first runs another request, whose rows a new one must not see."""
+    passes, the ring's wrap (past 80 frames) and requests after a reset: the bits of
+    one frame at a time, whose first frames are the oracle's. The state first runs
+    another request, whose rows a new one must not see."""
     mimi_w, convs = random_mimi(911), random_pcm_convs(912)
     frames = sum(counts)
     x = np.random.default_rng(913).standard_normal((frames, 32)).astype(np.float32)
