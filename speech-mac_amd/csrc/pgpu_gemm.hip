@@ -20,15 +20,15 @@ __global__ __launch_bounds__(kTaskThreads) void k_gemm_wide(GemmArgs a) {
     gemm_wide_task<SRC, EPI, Q8>(a, blockIdx.x, blockIdx.y, (uint16_t *)bsh4, NoWait{});
 }
 
-// gemm_split_task on fp32 rows (a.ln_x, [streams][k_cols]): a lane splits its
-// 8 columns of each block itself, all 8 blocks of its wave's range (K = 2048)
-// requested at once. Every row tile's work-group splits the rows again, which
-// is less than the launch that would do it for them: a 512 x 2048 product of
-// one row is bound by its launches and load latencies (7.5 us with the rows
-// split by a launch of their own, 5.2 with this).
-template <bool Q8>
+// gemm_split_task on fp32 rows (a.ln_x, [streams][k_cols]) and Q8 weights: a lane
+// splits its 8 columns of each block itself, CH blocks of its wave's range
+// requested at once (all of them up to K = 2048). Every row tile's work-group
+// splits the rows again, which is less than the launch that would do it for them
+// as long as the work-groups run at once: a 512 x 2048 product of one row is bound
+// by its launches and load latencies (7.5 us with the rows split by a launch of
+// their own, 5.2 with this).
+template <int CH>
 __global__ __launch_bounds__(kTaskThreads) void k_gemm_rows(GemmArgs a) {
-    constexpr int CH = 8;
     __shared__ f32x4 partial[kTaskWaves * 64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, tile = blockIdx.x, st = blockIdx.y;
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(kTaskThreads) void k_gemm_rows(GemmArgs a) {
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     bool bad = false;
     for (int kb0 = kb_begin; kb0 < kb_end; kb0 += CH) {
-        WChunk<Q8, CH> w;
+        WChunk<true, CH> w;
         load_weights(w, a, tile, kbn, lane, kb0, kb_end);
         float4 x[CH][2];
 #pragma unroll
@@ -167,16 +167,22 @@ extern "C" int pgpu_gemm_store_rows(void *stream, const pgpu_matrix *w, const fl
                                     int streams, float *out, int ld_out, int *status) {
     GemmArgs a;
     const pgpu_gemm_input in = {.rows = rows};
-    if (!w || !rows || !out || !status || streams <= 0 || !w->rows || w->rows % 16 ||
+    if (!w || !w->q8 || !rows || !out || !status || streams <= 0 || !w->rows || w->rows % 16 ||
         !w->columns || w->columns % 32 || !base_args(a, w, &in, streams, status))
         return bad_arguments("pgpu_gemm_store_rows");
     a.out = out;
     a.ld_out = ld_out;
     const dim3 grid(a.n_rows / 16, (streams + 15) / 16);
-    if (w->q8)
-        hipLaunchKernelGGL(k_gemm_rows<true>, grid, dim3(kTaskThreads), 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL(k_gemm_rows<false>, grid, dim3(kTaskThreads), 0, (hipStream_t)stream, a);
+    // A wave's blocks in equal chunks of at most 8 (a block past its range costs
+    // what a block costs).
+    const int per = (a.k_cols / 32 + kTaskWaves - 1) / kTaskWaves, chunks = (per + 7) / 8;
+    const int ch = (per + chunks - 1) / chunks;
+    const auto k = ch <= 1   ? k_gemm_rows<1>
+                   : ch <= 2 ? k_gemm_rows<2>
+                   : ch <= 4 ? k_gemm_rows<4>
+                   : ch <= 6 ? k_gemm_rows<6>
+                             : k_gemm_rows<8>;
+    hipLaunchKernelGGL(k, grid, dim3(kTaskThreads), 0, (hipStream_t)stream, a);
     return launch_ok("pgpu_gemm_store_rows");
 }
 

@@ -84,6 +84,9 @@ const float *ph_rope_table(float theta);
 enum { PH_ROPE_LONG_ROWS = 8192 * 16 };
 const float *ph_rope_table_long(float theta);
 
+/* phonon_q8_device_matvec's route at a width other than 512. */
+int ph_q8_one_launch(size_t rows, size_t columns, size_t batch);
+
 int ph_all_finite(const float *values, size_t count);
 int ph_overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes);
 

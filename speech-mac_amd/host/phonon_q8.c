@@ -103,6 +103,23 @@ int phonon_q8_device_create(const PhononQ8Block *weights, size_t rows, size_t co
     return 1;
 }
 
+/* Whether a product of a width other than 512 splits its rows in every row tile's
+ * work-group (one launch) or by a launch of their own. The second takes 6.4 us
+ * at least, the first is short while its work-groups run at once: their number
+ * times the width, a partly filled tile of 16 rows counting half of what it lacks.
+ * us, two launches / one: 512 x 2048 1 row 7.1 / 5.1, 64 rows 9.0 / 6.9; 4096 x
+ * 2048 17 rows (12.8 M) 10.6 / 9.5, 32 rows (16.8 M) 11.0 / 11.5; 6144 x 2048 8
+ * rows (9.4 M) 10.1 / 9.0, 16 rows (12.6 M) 10.5 / 11.4; 8192 x 1024 17 rows (12.8 M)
+ * 10.4 / 10.3, 32 rows (16.8 M) 10.7 / 11.9; 16384 x 1024 1 row (8.9 M) 9.6 / 8.1,
+ * 64 rows (67 M) 27.4 / 39.6; 4096 x 4096 8 rows (12.6 M) 10.4 / 10.3, 16 rows (16.8 M)
+ * 11.8 / 12.6. One block a wave (up to 256 columns) is always faster: 16384 x 128, 64
+ * rows 18.6 / 7.5. Past 4096 columns a wave takes several rounds of loads: 512 x 8192
+ * 8 rows 14.5 / 15.3, 16 rows 16.7 / 19.9. */
+int ph_q8_one_launch(size_t rows, size_t columns, size_t batch) {
+    const size_t tiles = (batch + 15) / 16, work = rows / 16 * (16 * tiles + batch) / 2;
+    return columns <= 256 || (columns <= 4096 && work * columns <= 13000000);
+}
+
 int phonon_q8_device_matvec(PhononQ8Device *m, size_t copy, const float *x, float *y,
                             size_t batch, void *stream) {
     /* The kernels read x and write y 16 bytes at a time. */
@@ -117,9 +134,10 @@ int phonon_q8_device_matvec(PhononQ8Device *m, size_t copy, const float *x, floa
         const pgpu_gemm_input rows = {.rows = x};
         return pgpu_gemm_store(stream, w, &rows, (int)batch, NULL, y, (int)w->rows, m->status);
     }
-    /* One launch for other widths too; an output that overlaps the input needs
-     * the rows read before any result is written. */
-    if (!ph_overlap(x, batch * w->columns * sizeof(float), y, batch * w->rows * sizeof(float)))
+    /* An output that overlaps the input needs the rows read before any result is
+     * written. */
+    if (ph_q8_one_launch(w->rows, w->columns, batch) &&
+        !ph_overlap(x, batch * w->columns * sizeof(float), y, batch * w->rows * sizeof(float)))
         return pgpu_gemm_store_rows(stream, w, x, (int)batch, y, (int)w->rows, m->status);
     const pgpu_gemm_input in = {.split = m->xs};
     return pgpu_split_rows(stream, x, (int)batch, (int)w->columns, m->xs, m->status) &&

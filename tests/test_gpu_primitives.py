@@ -154,11 +154,14 @@ def test_q8_device_matvec_512_columns_rows_path(lib, oracle, syn, pkg, batch):
 
 
 @pytest.mark.parametrize("rows,cols,batch", [
-    (16, 32, 1), (48, 64, 3), (512, 2048, 16), (512, 2048, 17), (32, 2080, 2), (64, 4128, 33)])
+    (16, 32, 1), (48, 64, 3), (512, 2048, 16), (512, 2048, 17), (32, 2080, 2), (64, 4128, 33),
+    (32, 256, 64), (64, 288, 5), (48, 1024, 16), (48, 1056, 17), (16, 1536, 33), (32, 2816, 3),
+    (32, 4096, 48), (8192, 1024, 17), (8192, 1024, 32)])
 def test_q8_device_matvec_rows_split_in_the_product(lib, syn, pkg, rows, cols, batch):
-    """Widths other than 512 split their rows inside the product: block counts
-    below, at and past the eight a wave requests at once, odd ones, and whole and
-    partial 16-row tiles. The bits of the rows split by a launch of their own,
+    """Widths other than 512 split their rows inside the product: each number of
+    blocks that a wave requests at once (1, 2, 4, 6, 8), ranges of one and several
+    such rounds, odd ones, whole and partial 16-row tiles, and both sides of the line
+    to a launch of the rows' own. The bits of the rows split by a launch of their own,
     which an output laid over the input still takes; a non-finite input is
     reported."""
     rng = np.random.default_rng(rows + cols)
