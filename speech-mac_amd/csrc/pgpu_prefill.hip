@@ -496,15 +496,19 @@ __global__ __launch_bounds__(kTaskThreads) void k_prefill_split(GemmArgs a, int 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int chain = wave / kWr, wr = wave % kWr;
-    // Position groups over the XCDs, as in k_prefill_gemm.
+    // A position group's work-groups on one XCD, as in k_prefill_gemm, eight such
+    // groups at a time; the last pos_groups % 8 go over all of them. (Only counts
+    // that 8 divides went by XCD before, 16 prompts of 200 positions, whose MLP-out
+    // product has 100 groups, took 1593 us a call; of 192, with 96, 1384. Now 1516; 16 of 72 980 -> 909.)
+    const int whole = pos_groups & ~7, id = blockIdx.x - whole * row_groups;
     int row_group, pos_group;
-    if (pos_groups % 8 == 0) {
+    if (id < 0) {
         const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
         pos_group = xcd + 8 * (local / row_groups);
         row_group = local % row_groups;
     } else {
-        pos_group = blockIdx.x / row_groups;
-        row_group = blockIdx.x % row_groups;
+        pos_group = whole + id / row_groups;
+        row_group = id % row_groups;
     }
     const int pt0 = pos_group * PW, rt0 = (row_group * kWr + wr) * RW;
     const int last_tile = (a.streams - 1) >> 4, kb0 = chain * kChain;
@@ -1403,13 +1407,14 @@ int launch_split(const GemmArgs &a, hipStream_t stream) {
 //   out         5.8 / 10.0   6.0 / 10.1   7.5 / 10.4  12.5 / 11.0
 //   MLP in     12.7 / 22.9  11.8 / 22.9  19.2 / 24.2  27.6 / 25.4
 //   MLP out    10.0 / 25.4   9.8 / 25.6  16.8 / 25.8  24.0 / 26.7
-// (4096 rows: MLP out 31.2 / 29.9.) Within that: the smallest tile whose
+// (4096 rows: MLP out 31.2 / 29.9; a whole call of 3072 positions 1379 / 1399, of
+// 3200 1516 / 1472.) Within that: the smallest tile whose
 // work-groups still run at once, one per CU, since a work-group's time is
 // mostly the latency of its loads (24 rows, QKV: 4.8 with 1 x 1 tiles a wave,
 // 6.7 with 2 x 1, 7.5 with 2 x 2; 400 rows: 9.1, 8.8, 8.3).
 template <int EPI>
 constexpr int split_tiles(bool k2048) {
-    return EPI == EPI_QKV ? 80 : EPI == EPI_GELU_SPLIT ? 144 : k2048 ? 200 : 128;
+    return EPI == EPI_QKV ? 80 : EPI == EPI_GELU_SPLIT ? 144 : k2048 ? 192 : 128;
 }
 
 template <int EPI, bool SCALED>

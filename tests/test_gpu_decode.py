@@ -916,11 +916,12 @@ def test_fast_prefill_around_the_short_prompt_path(lib, syn, pkg, counts, first)
 @pytest.mark.parametrize("counts,first", [
     ([1], [0]), ([17, 3], [0, 5]), ([129], [0]), ([250, 91], [0, 33]), ([40, 16], [4190, 63]),
     ([70] * 15, [1] * 15), ([70] * 16, [1] * 16), ([1281], [0]), ([2049], [0]), ([2320], [0]),
-    ([3216], [0])])
+    ([2432], [0]), ([3072], [0]), ([3088], [0]), ([3216], [0])])
 def test_fast_prefill_tiles_and_runs(lib, syn, pkg, counts, first):
     """Calls on both sides of the fast prefill's choices: one position and
     ragged tails, each projection tile (wave tiles of 1 x 1, 2 x 1 and 2 x 2,
-    and where the many-position kernels take over), short attention runs over
+    position groups that eight XCDs divide and that they do not, and where the
+    many-position kernels take over), short attention runs over
     contexts of more than 64 blocks a wave, 15 and 16 pairs of long runs. The
     exact prefill of the same call is the reference: every row within 1e-4
     normwise."""
