@@ -1340,8 +1340,8 @@ __global__ __launch_bounds__(64 * kShortWaves) void k_prefill_attention_short(
     for (int r = 0; r < 4; r++)
         part[wave][r][lane] = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
     __syncthreads();
-    // Waves 0 .. 3: wave w finishes dimensions 16 g + 4 w .. + 3.
-    if (wave >= 4) return;
+    // Wave w finishes dimensions 16 g + 4 w .. + 3.
+    static_assert(kShortWaves == 4, "a wave for each quarter of a lane's dimensions");
     float top = red[0][0][n];
 #pragma unroll
     for (int w = 1; w < kShortWaves; w++) top = fmaxf(top, red[0][w][n]);

@@ -1126,12 +1126,23 @@ def test_one_launch_step_equals_phase_launches(lib, syn, pkg, streams):
             assert np.array_equal(a, b)
 
 
+def step_tasks(lib, bt):
+    """The one-launch step's task list."""
+    n = lib.phonon_flow_batch_schedule(bt.batch, None, 0)
+    out = np.zeros(n, np.uint32)
+    u32 = out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))
+    assert lib.phonon_flow_batch_schedule(bt.batch, u32, n) == n
+    return out
+
+
 @pytest.mark.parametrize("streams,high", [(12, 200), (12, 1200), (24, 4000), (40, 200), (70, 900),
                                           (96, 4000)])
 def test_schedule_follows_the_contexts(lib, syn, pkg, streams, high):
     """The default step lists one or two attention splits per task and places a
     tile's chain by the contexts: few and many splits for one tile, for several,
-    and past the line to two per task. The bits of the layers phase by phase."""
+    and past the line to two per task. Its list is the one that the rules give for
+    these contexts (each stream's splits 256 positions ahead), its results the bits
+    of the layers phase by phase."""
     layers = 2
     model, views = scaled_model(syn, 185, layers), pkg.Views()
     w = views.layers(model)
@@ -1153,6 +1164,22 @@ def test_schedule_follows_the_contexts(lib, syn, pkg, streams, high):
             y = np.zeros((streams, 512), np.float32)
             assert lib.phonon_flow_batch_step(bt.batch, fp(x), 10000.0, fp(y)), pkg.last_error(lib)
             outs.append(y.view(np.uint32))
+        if flow:
+            got = step_tasks(lib, bt)
+            cover = np.minimum((lengths + 512) // 256, -(-16 * table_len // 256))
+            size = ctypes.c_size_t
+            rounds = lib.ph_flow_step_rounds(size(streams), size(int(cover.sum())))
+            units = -(-cover.astype(np.int64) // rounds)
+            lib.ph_flow_step_placement.restype = pkg.PgpuFlowPlacement
+            place = lib.ph_flow_step_placement(size(-(-streams // 16)),
+                                               size(int(units.sum()) * rounds * 8), rounds)
+            units = units.astype(np.uintp)
+            want = np.zeros(got.size, np.uint32)
+            assert lib.pgpu_flow_schedule(
+                streams, layers, units.ctypes.data_as(ctypes.POINTER(ctypes.c_size_t)),
+                ctypes.byref(place), 0, want.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)),
+                want.size) == got.size
+            assert np.array_equal(got, want)
         bt.close()
     assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[3])
 
@@ -1186,27 +1213,20 @@ def test_schedule_follows_contexts_that_shrink(lib, syn, pkg):
             assert lib.phonon_flow_batch_step(bt.batch, fp(x), 10000.0, fp(y)), pkg.last_error(lib)
         return y
 
-    def tasks(bt):
-        n = lib.phonon_flow_batch_schedule(bt.batch, None, 0)
-        out = np.zeros(n, np.uint32)
-        u32 = out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))
-        assert lib.phonon_flow_batch_schedule(bt.batch, u32, n) == n
-        return out
-
     bt, tables = batch()
     expected = run(bt, tables, short, 1)
-    fresh = tasks(bt)
+    fresh = step_tasks(lib, bt)
     bt.close()
     bt, tables = batch()
     run(bt, tables, long, 1)
-    whole = tasks(bt)
+    whole = step_tasks(lib, bt)
     assert whole.size > fresh.size
     for lengths in (short, long, short, long):
         run(bt, tables, lengths, 1)
-        assert np.array_equal(tasks(bt), whole)
+        assert np.array_equal(step_tasks(lib, bt), whole)
     run(bt, tables, long, 4)
     got = run(bt, tables, short, 1)
-    assert np.array_equal(tasks(bt), fresh)
+    assert np.array_equal(step_tasks(lib, bt), fresh)
     assert np.array_equal(got.view(np.uint32), expected.view(np.uint32))
     bt.close()
 
